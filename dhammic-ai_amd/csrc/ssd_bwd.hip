@@ -51,9 +51,14 @@ __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const
   // thread t moves position t's four values with one 16-byte access through LDS (the per-head
   // 4-byte accesses touch a line per lane, four times as many L2 requests)
   __shared__ float s_dt[4][256], s_ddt[4][256];
+  // Two kernel heads per caller head (d.hs): the block's four heads are two caller heads, whose ddt and
+  // per-token da are summed through LDS; a wave past the last head repeats it (same values, no output of
+  // its own), so that every wave meets the barriers.
+  __shared__ float s_da[4][256];
   const int c = blockIdx.x;
   const int w = threadIdx.x >> 6;
-  const int h = blockIdx.y * 4 + w;
+  const int hs = d.hs;
+  const int h = hs ? min((int)blockIdx.y * 4 + w, d.H - 1) : blockIdx.y * 4 + w;
   const int lane = lane_id();
   if (h >= d.H) return;  // never taken when H % 4 == 0 (every wave of the block then has a head)
   const ChunkInfo ci = chunks[c];
@@ -63,7 +68,7 @@ __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const
     return;
   }
   const bool vec_dt = d.a_mode == 0 && d.has_dt && (d.H & 3) == 0 && (reinterpret_cast<uintptr_t>(dt) & 15) == 0;
-  const bool vec_ddt = vec_dt && ddt != nullptr && (reinterpret_cast<uintptr_t>(ddt) & 15) == 0;
+  const bool vec_ddt = !hs && vec_dt && ddt != nullptr && (reinterpret_cast<uintptr_t>(ddt) & 15) == 0;
   if (vec_dt) {
     const int tp = threadIdx.x;  // position; Qpad <= 256 = blockDim.x
     floatx4 q = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -146,11 +151,16 @@ __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const
     const int64_t row = ci.row0 + l;
     if (d.a_mode == 0) {
       const float dtv = vec_dt ? s_dt[w][l] : (d.has_dt ? dt[row * d.H + h] : 1.0f);
-      if (vec_ddt) s_ddt[w][l] = t[e] + Ah[h] * da;
+      if (vec_ddt || hs) s_ddt[w][l] = (ddt && d.has_dt) ? t[e] + Ah[h >> hs] * da : 0.0f;
       else if (ddt && d.has_dt) ddt[row * d.H + h] = t[e] + Ah[h] * da;
       dAp += dtv * da;
     } else {
       // per-token decay (with dt: the trapezoidal mode's scan, where a does not depend on dt)
+      if (hs) {
+        s_da[w][l] = da;
+        s_ddt[w][l] = (ddt && d.has_dt) ? t[e] : 0.0f;
+        continue;
+      }
       if (dA_tok) dA_tok[row * d.H + h] = from_f<T>(da);
       if (da32) da32[row * d.H + h] = da;
       if (ddt && d.has_dt) ddt[row * d.H + h] = t[e];
@@ -158,6 +168,21 @@ __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const
   }
   for (int o = 32; o > 0; o >>= 1) dAp += __shfl_xor(dAp, o, 64);
   if (lane == 0) bf.dA_part[ch] = dAp;
+  if (hs) {
+    __syncthreads();
+    const int tp = threadIdx.x, Hr = d.H >> 1;
+    for (int q = 0; q < 2; ++q) {
+      const int hr = blockIdx.y * 2 + q;
+      if (tp >= ci.len || hr >= Hr) break;
+      const int64_t o = (ci.row0 + tp) * (int64_t)Hr + hr;
+      if (ddt && d.has_dt) ddt[o] = s_ddt[2 * q][tp] + s_ddt[2 * q + 1][tp];
+      if (d.a_mode != 0) {
+        const float da = s_da[2 * q][tp] + s_da[2 * q + 1][tp];
+        if (dA_tok) dA_tok[o] = from_f<T>(da);
+        if (da32) da32[o] = da;
+      }
+    }
+  }
   if (vec_ddt) {
     __syncthreads();
     const int tp = threadIdx.x;

@@ -25,7 +25,7 @@ struct Plan {
   int64_t nslices, hslice, npass_blk, norm_blocks;
   // byte offsets inside each workspace
   size_t o_chunks, o_seq0, o_cs, o_bfac, o_ffac, o_ffac2, o_fast, o_hin, o_hinlo, o_ypre, o_rstd, o_tzdt, o_tzrho, o_tzgam,
-      o_tzcb, o_Dtok, o_hgam, o_hgamlo, saved_bytes;
+      o_tzcb, o_Dtok, o_hgam, o_hgamlo, o_dtrep, o_Drep, saved_bytes;
   size_t o_st, fwd_bytes;
   size_t o_dyp, o_dst, o_dtot, o_rowG, o_colG, o_eterm, o_dcs, o_xdx, o_dD, o_dA, o_dBp, o_dCp, o_dw, o_dS, o_dSf, o_dst16,
       o_xdy, o_tzddt, o_tzda, bwd_bytes;
@@ -33,7 +33,8 @@ struct Plan {
   int rows_chunk;  // fused path: the chunk-resident row kernel (k_bwd_rows) instead of k_bwd_gemm
 };
 
-int plan(const ssd_desc_t* s, Plan* p) {
+// `split`: whether a wide bf16 head may run as two heads of half its width (below).
+int plan(const ssd_desc_t* s, Plan* p, bool split = true) {
   if (!s || !p) return SSD_ERR_INVALID;
   memset(p, 0, sizeof(*p));
   if (s->batch < 1 || s->seqlen < 1 || s->nheads < 1 || s->headdim < 1 || s->ngroups < 1 || s->dstate < 1 ||
@@ -74,6 +75,15 @@ int plan(const ssd_desc_t* s, Plan* p) {
   SsdDims& d = p->d;
   d.batch = (int)s->batch; d.seqlen = (int)s->seqlen; d.H = (int)s->nheads; d.P = (int)s->headdim;
   d.G = (int)s->ngroups; d.N = (int)s->dstate; d.Q = (int)s->chunk;
+  // The fused bf16 kernels hold heads of up to 64 columns. A head's P channels are independent given its dt,
+  // A, B, C and D, so a wider one whose half is a whole number of 16-byte vectors runs as two kernel heads of
+  // P / 2 that share them: x, y, z, the states and their gradients keep their layout (heads are the slower
+  // dimension), the cumsum launch repeats dt and D, and the finish sums the gradients of the pair.
+  if (split && s->dtype == SSD_DTYPE_BF16 && d.P > 64 && d.P % 16 == 0 && d.N % 8 == 0 && 2 * s->nheads <= kMaxGrid) {
+    d.H *= 2;
+    d.P /= 2;
+    d.hs = 1;
+  }
   // feature widths padded to 32, 64 or 128 (the tile shapes the kernels are built for)
   d.Ppad = d.P <= 32 ? 32 : (d.P <= 64 ? 64 : 128);
   d.Npad = d.N <= 32 ? 32 : (d.N <= 64 ? 64 : 128);
@@ -148,6 +158,8 @@ int plan(const ssd_desc_t* s, Plan* p) {
   p->o_tzcb = d.trapz ? take((size_t)R * d.G * sizeof(float)) : 0;
   p->o_hgam = d.trapz == SSD_TRAPZ_DROP_BETA_DA ? take(MC * H * PN * es) : 0;
   p->o_hgamlo = (d.trapz == SSD_TRAPZ_DROP_BETA_DA && lo) ? take(MC * H * PN) : 0;
+  p->o_dtrep = (d.hs && d.has_dt && !d.trapz) ? take(rh) : 0;
+  p->o_Drep = (d.hs && d.has_D) ? take(H * sizeof(float)) : 0;
   p->saved_bytes = off;
   off = 0;
   p->o_st = take(MC * H * PN * sizeof(float));
@@ -203,6 +215,8 @@ void bind_saved(const Plan& p, void* saved, SsdBufs* b) {
   b->nrowg = p.nrowg;
   b->ndcs = p.fused_bwd && !p.rows_chunk ? 2 : 1;
   b->rows_chunk = p.rows_chunk;
+  b->dt_rep = p.o_dtrep ? reinterpret_cast<float*>(s + p.o_dtrep) : nullptr;
+  b->D_rep = p.o_Drep ? reinterpret_cast<float*>(s + p.o_Drep) : nullptr;
   if (p.d.trapz) {
     b->tz_dt = reinterpret_cast<float*>(s + p.o_tzdt);
     b->tz_rho = reinterpret_cast<float*>(s + p.o_tzrho);
@@ -280,11 +294,8 @@ struct PhaseTimer {
     SSD_TRY((tm).end(ph));        \
   } while (0)
 
-int fwd_impl(const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* saved, size_t saved_bytes, void* scratch,
+int fwd_impl(Plan& p, const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* saved, size_t saved_bytes, void* scratch,
              size_t scratch_bytes, void* stream) {
-  Plan p;
-  int st = plan(desc, &p);
-  if (st != SSD_OK) return st;
   SsdDims& d = p.d;
   if (!a || !a->x || !a->A || !a->B || !a->C || !a->y) return SSD_ERR_INVALID;
   if ((d.has_dt && !d.trapz && !a->dt) || (d.has_D && !a->D) || (d.has_z && (!a->z || !a->norm_weight)) ||
@@ -300,22 +311,24 @@ int fwd_impl(const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* saved, size_
   b.st = reinterpret_cast<float*>(scratch);
   b.fwd_fac = reinterpret_cast<float*>(static_cast<unsigned char*>(scratch) + p.o_ffac);
   b.fwd_fac2 = p.o_ffac2 ? reinterpret_cast<float*>(static_cast<unsigned char*>(scratch) + p.o_ffac2) : nullptr;
-  // trapezoidal mode: the scan's dt is gamma + rho, written by the coefficient kernel
-  const float* dt = d.trapz ? b.tz_dt : a->dt;
-  SsdIn in = {a->x, dt, a->A, a->B, a->C, a->D, a->z, a->norm_weight, a->init, a->cu_seqlens};
+  // trapezoidal mode: the scan's dt is gamma + rho, written by the coefficient kernel; dt and D per kernel
+  // head where a caller head is two of them
+  const float* dt = d.trapz ? b.tz_dt : (b.dt_rep ? b.dt_rep : a->dt);
+  const float* Dk = b.D_rep ? b.D_rep : a->D;
+  SsdIn in = {a->x, dt, a->A, a->B, a->C, Dk, a->z, a->norm_weight, a->init, a->cu_seqlens};
   const PhaseTimer tm{a->events, s};
   const bool fused_state = state_fused_supported(p.dtype, d);
   // packed sequences: the chunk table from cu_seqlens; fixed-length batches: written by the cumsum launch
   if (d.varlen) SSD_PHASE(tm, SSD_PH_CHUNK_TABLE, launch_chunk_table(d, b, a->cu_seqlens, s));
   SSD_PHASE(tm, SSD_PH_CUMSUM,
-            launch_chunk_cumsum(p.dtype, d, b, a->A, dt, desc->want_A_cumsum ? a->A_cumsum_out : nullptr, s));
+            launch_chunk_cumsum(p.dtype, d, b, a->A, a->dt, a->D, desc->want_A_cumsum ? a->A_cumsum_out : nullptr, s));
   // the factorised forward scan (bf16, 16-byte rows) computes S = C B^T per chunk and group anyway: in the
   // trapezoidal mode it also writes the per-token cb = C_t . B_t (S's diagonal) and D per token
   const bool fwd_fact = scan_fwd_chunk_supported(p.dtype, d) && d.vec_x && d.vec_bc;
   b.tz_cb_fwd = d.trapz && fwd_fact ? 1 : 0;
   if (d.trapz) {
     SSD_TRY(tm.begin(SSD_PH_TRAPZ_PREP));
-    SSD_TRY(launch_trapz_prep(p.dtype, d, b, a->A, a->gamma, a->beta, a->B, a->C, a->D, a->cu_seqlens, s));
+    SSD_TRY(launch_trapz_prep(p.dtype, d, b, a->A, a->gamma, a->beta, a->B, a->C, Dk, a->cu_seqlens, s));
     if (d.trapz == SSD_TRAPZ_DROP_BETA_DA && !fused_state) {
       // the gamma path's own states, for the backward's gamma-path decay gradient (the fused walk computes
       // them in the scan's forward walk launch)
@@ -346,7 +359,7 @@ int fwd_impl(const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* saved, size_
     // factorised decay, then the exact kernel on the (chunk, head) pairs it cannot take
     SSD_TRY(tm.begin(SSD_PH_FWD_SCAN));
     SSD_TRY(launch_scan_fwd_fact(d, b, in, yout, s));
-    if (b.tz_cb_fwd) SSD_TRY(launch_trapz_dtok(d, b, a->D, s));
+    if (b.tz_cb_fwd) SSD_TRY(launch_trapz_dtok(d, b, Dk, s));
     SSD_TRY(launch_scan_fwd_chunk(d, b, in, yout, b.fast, s));
     SSD_TRY(tm.end(SSD_PH_FWD_SCAN));
   } else
@@ -417,19 +430,27 @@ size_t ssd_workspace_bytes(const ssd_desc_t* desc, int kind) {
 
 int ssd_fwd(const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* saved, size_t saved_bytes, void* scratch,
             size_t scratch_bytes, void* stream) {
-  return fwd_impl(desc, a, saved, saved_bytes, scratch, scratch_bytes, stream);
+  Plan p;
+  const int st = plan(desc, &p);
+  if (st != SSD_OK) return st;
+  return fwd_impl(p, desc, a, saved, saved_bytes, scratch, scratch_bytes, stream);
 }
 
 int ssd_fwd_noalloc(const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* stream) {
   Plan p;
-  const int st = plan(desc, &p);
+  int st = plan(desc, &p);
   if (st != SSD_OK) return st;
-  // both forward workspaces, one after the other (the saved part is not kept for a backward)
+  // both forward workspaces, one after the other (the saved part is not kept for a backward); a wide head's
+  // pair takes a little more of it than the head itself, so near the limit the head runs whole
+  if (p.d.hs && align_up(p.saved_bytes) + p.fwd_bytes > (size_t)SSD_NOALLOC_SCRATCH_BYTES) {
+    st = plan(desc, &p, false);
+    if (st != SSD_OK) return st;
+  }
   const size_t off = align_up(p.saved_bytes);
   if (off + p.fwd_bytes > (size_t)SSD_NOALLOC_SCRATCH_BYTES) return SSD_ERR_TOO_LARGE;
   unsigned char* base = static_cast<unsigned char*>(scratch_on_current_device());
   if (!base) return SSD_ERR_HIP;
-  return fwd_impl(desc, a, base, p.saved_bytes, base + off, p.fwd_bytes, stream);
+  return fwd_impl(p, desc, a, base, p.saved_bytes, base + off, p.fwd_bytes, stream);
 }
 
 int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, size_t saved_bytes, void* scratch,
@@ -449,8 +470,8 @@ int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, 
   memset(&b, 0, sizeof(b));
   bind_saved(p, const_cast<void*>(saved), &b);
   bind_bwd(p, scratch, &b);
-  const float* dt = d.trapz ? b.tz_dt : a->dt;
-  SsdIn in = {a->x, dt, a->A, a->B, a->C, a->D, a->z, a->norm_weight, a->init, a->cu_seqlens};
+  const float* dt = d.trapz ? b.tz_dt : (b.dt_rep ? b.dt_rep : a->dt);
+  SsdIn in = {a->x, dt, a->A, a->B, a->C, b.D_rep ? b.D_rep : a->D, a->z, a->norm_weight, a->init, a->cu_seqlens};
   const PhaseTimer tm{a->events, s};
   // the fused backward needs 16-byte vector access; otherwise the column / row kernels run
   const bool fused = p.fused_bwd && d.vec_x && d.vec_bc;

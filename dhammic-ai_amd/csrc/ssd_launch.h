@@ -25,7 +25,7 @@ struct SsdIn {
 // packed sequences (d.varlen) only: a fixed-length batch's table is written by launch_chunk_cumsum
 hipError_t launch_chunk_table(const SsdDims& d, const SsdBufs& b, const int32_t* cu, hipStream_t s);
 hipError_t launch_chunk_cumsum(int dtype, const SsdDims& d, const SsdBufs& b, const void* A,
-                               const float* dt, void* A_cumsum_out, hipStream_t s);
+                               const float* dt, const float* D, void* A_cumsum_out, hipStream_t s);
 hipError_t launch_decay_chunk(int dtype, int batch, int H, int nch, int Q, const void* Acs,
                               void* out, hipStream_t s);
 hipError_t launch_materialize_L(int dtype, int batch, int seqlen, int H, int Q, const void* a,

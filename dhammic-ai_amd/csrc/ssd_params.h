@@ -22,6 +22,10 @@ struct SsdDims {
   // 16-byte global loads allowed for x/dy/z-shaped tensors and for B/C (set per call
   // from the feature widths and the pointers' alignment)
   bool vec_x, vec_bc;
+  // log2 of the kernel heads per caller head: 1 where a bf16 head wider than 64 runs as two heads of half its
+  // width (plan() in ssd_capi.hip). H, P and hpg are then the kernels' (2 H heads of P / 2); the caller's
+  // per-head tensors (dt, A, D, gamma, beta and their gradients) have H >> hs heads.
+  int hs;
 };
 
 // Internal buffers (all inside the caller's workspaces).
@@ -78,6 +82,9 @@ struct SsdBufs {
   float* tz_gam;           // [R][H]
   float* tz_cb;            // [R][G]
   float* Dtok;             // [R][H] (nullptr outside trapezoidal mode)
+  // hs = 1 (saved): the caller's dt and D per kernel head, written by the cumsum launch
+  float* dt_rep;           // [R][H]
+  float* D_rep;            // [H]
   int tz_cb_fwd;           // 1: cb and Dtok are written by the factorised forward scan (the diagonal of its
                            // C B^T units), not by the trapezoidal prep kernels
   void* hgam;              // [max_chunks][H][Ppad][Npad] (T)

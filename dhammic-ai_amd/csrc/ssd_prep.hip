@@ -94,7 +94,8 @@ hipError_t launch_chunk_table(const SsdDims& d, const SsdBufs& b, const int32_t*
 // ffac = exp(clamp(cs_last - cs_t)) dt_t (trapezoidal mode: zeros here, the
 // coefficient kernel writes the chunk's positions with its own dt), ffac2
 // (trapezoidal gamma walk: zeros here likewise). For a fixed-length batch it
-// also writes the chunk table (no k_chunk_table launch).
+// also writes the chunk table (no k_chunk_table launch). With two kernel heads per caller head (d.hs) it
+// also writes dt and D per kernel head.
 // ---------------------------------------------------------------------------
 // One row of Qpad fp32 values, `per` consecutive positions per lane: a 16-byte store per lane when
 // each lane holds four and the row is 16-byte aligned.
@@ -112,12 +113,15 @@ __global__ void __launch_bounds__(256) k_chunk_cumsum(SsdDims d, ChunkInfo* __re
                                                       const void* __restrict__ Av, const float* __restrict__ dt,
                                                       float* __restrict__ cs, T* __restrict__ acs_out,
                                                       int32_t* __restrict__ fast, float* __restrict__ ffac,
-                                                      float* __restrict__ ffac2, float* __restrict__ bfac) {
+                                                      float* __restrict__ ffac2, float* __restrict__ bfac,
+                                                      float* __restrict__ dt_rep, const float* __restrict__ Dv,
+                                                      float* __restrict__ D_rep) {
   // dt of the block's four heads, [head][position] (Qpad <= 256)
   __shared__ float s_dt[4][256];
   const int c = blockIdx.x;
   const int h0 = blockIdx.y * 4, hw = threadIdx.x >> 6;
   const int h = h0 + hw;
+  const int hs = d.hs, Hr = d.H >> hs, hr = h >> hs;  // the caller's heads
   const int lane = lane_id();
   ChunkInfo ci;
   if (build_table) {
@@ -146,8 +150,13 @@ __global__ void __launch_bounds__(256) k_chunk_cumsum(SsdDims d, ChunkInfo* __re
     if (l < d.Qpad) {
       float q[4] = {1.0f, 1.0f, 1.0f, 1.0f};
       if (l < ci.len) {
-        const float* p = dt + ((int64_t)ci.row0 + l) * d.H + h0;
-        if ((d.H & 3) == 0 && (reinterpret_cast<uintptr_t>(dt) & 15) == 0) {
+        const float* p = dt + ((int64_t)ci.row0 + l) * Hr + (h0 >> hs);
+        if (hs) {
+          // two kernel heads per caller head: their dt per kernel head goes out for the scan kernels
+          float* o = dt_rep + ((int64_t)ci.row0 + l) * d.H + h0;
+          for (int k = 0; k < 4; ++k)
+            if (h0 + k < d.H) o[k] = q[k] = p[k >> 1];
+        } else if ((d.H & 3) == 0 && (reinterpret_cast<uintptr_t>(dt) & 15) == 0) {
           const float4 f = *reinterpret_cast<const float4*>(p);
           q[0] = f.x; q[1] = f.y; q[2] = f.z; q[3] = f.w;
         } else {
@@ -160,6 +169,7 @@ __global__ void __launch_bounds__(256) k_chunk_cumsum(SsdDims d, ChunkInfo* __re
     __syncthreads();
   }
   if (h >= d.H) return;
+  if (D_rep && c == 0 && lane == 0) D_rep[h] = Dv[hr];
   const int per = d.Qpad / 64;  // 1 to 4 consecutive positions per lane
   float v[4] = {}, dtv[4] = {};
   float run = 0.0f;
@@ -172,17 +182,17 @@ __global__ void __launch_bounds__(256) k_chunk_cumsum(SsdDims d, ChunkInfo* __re
       const int nch = d.seqlen / d.Q;
       const T* A = reinterpret_cast<const T*>(Av);
       const int ll = min(l, ci.len - 1);
-      v[e] = to_f(A[(((int64_t)ci.seq * d.H + h) * nch + ci.idx_in_seq) * d.Q + ll]);
+      v[e] = to_f(A[(((int64_t)ci.seq * Hr + hr) * nch + ci.idx_in_seq) * d.Q + ll]);
       continue;
     }
     if (l < ci.len) {
       const int64_t row = ci.row0 + l;
       if (d.a_mode == 0) {
         const float* A = reinterpret_cast<const float*>(Av);
-        a = dtv[e] * A[h];
+        a = dtv[e] * A[hr];
       } else {
         const T* A = reinterpret_cast<const T*>(Av);
-        a = to_f(A[row * d.H + h]);
+        a = to_f(A[row * Hr + hr]);
       }
     }
     run += a;
@@ -237,9 +247,9 @@ __global__ void __launch_bounds__(256) k_chunk_cumsum(SsdDims d, ChunkInfo* __re
     const bool all_ok = __all(ok);
     if (lane == 0) fast[(int64_t)c * d.H + h] = all_ok ? 1 : 0;
   }
-  if (acs_out) {
+  if (acs_out && (h & ((1 << hs) - 1)) == 0) {
     const int nch = d.seqlen / d.Q;
-    T* o = acs_out + (((int64_t)ci.seq * d.H + h) * nch + ci.idx_in_seq) * d.Q;
+    T* o = acs_out + (((int64_t)ci.seq * Hr + hr) * nch + ci.idx_in_seq) * d.Q;
     for (int e = 0; e < per; ++e) {
       const int l = lane * per + e;
       if (l < d.Q) o[l] = from_f<T>(v[e]);
@@ -248,15 +258,17 @@ __global__ void __launch_bounds__(256) k_chunk_cumsum(SsdDims d, ChunkInfo* __re
 }
 
 hipError_t launch_chunk_cumsum(int dtype, const SsdDims& d, const SsdBufs& b, const void* A,
-                               const float* dt, void* A_cumsum_out, hipStream_t s) {
+                               const float* dt, const float* D, void* A_cumsum_out, hipStream_t s) {
   dim3 grid(d.max_chunks, (d.H + 3) / 4);
   const int build = d.varlen ? 0 : 1;  // fixed-length batches: the chunk table is written here
   if (dtype == 1)
     hipLaunchKernelGGL(k_chunk_cumsum<bf16>, grid, dim3(256), 0, s, d, b.chunks, b.seq_chunk0, build, A, dt, b.cs,
-                       reinterpret_cast<bf16*>(A_cumsum_out), b.fast, b.fwd_fac, b.fwd_fac2, b.bwd_fac);
+                       reinterpret_cast<bf16*>(A_cumsum_out), b.fast, b.fwd_fac, b.fwd_fac2, b.bwd_fac, b.dt_rep, D,
+                       b.D_rep);
   else
     hipLaunchKernelGGL(k_chunk_cumsum<float>, grid, dim3(256), 0, s, d, b.chunks, b.seq_chunk0, build, A, dt, b.cs,
-                       reinterpret_cast<float*>(A_cumsum_out), b.fast, b.fwd_fac, b.fwd_fac2, b.bwd_fac);
+                       reinterpret_cast<float*>(A_cumsum_out), b.fast, b.fwd_fac, b.fwd_fac2, b.bwd_fac, b.dt_rep, D,
+                       b.D_rep);
   return hipGetLastError();
 }
 

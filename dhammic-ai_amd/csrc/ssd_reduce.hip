@@ -73,9 +73,11 @@ __global__ void __launch_bounds__(1024) k_reduce_tail(SsdDims d, const ChunkInfo
       for (int c = t; c < d.max_chunks; c += 256) {
         const int len = chunks[c].len;
         if (len == 0) continue;
-        a += dA_part[(int64_t)c * d.H + h];
-        for (int j = 0; j < nrb; ++j)
-          if (j * SSD_BLK < len) dd += dD_part[((int64_t)c * d.H + h) * nrb + j];
+        for (int hk = h << d.hs; hk < (h + 1) << d.hs; ++hk) {  // the caller head's kernel heads
+          a += dA_part[(int64_t)c * d.H + hk];
+          for (int j = 0; j < nrb; ++j)
+            if (j * SSD_BLK < len) dd += dD_part[((int64_t)c * d.H + hk) * nrb + j];
+        }
       }
       ra[t] = a;
       rd[t] = dd;
@@ -110,7 +112,7 @@ __global__ void __launch_bounds__(1024) k_reduce_tail(SsdDims d, const ChunkInfo
 
 hipError_t launch_reduce_tail(const SsdDims& d, const SsdBufs& b, float* dA_head, float* dD, int nblocks, int width,
                               const float* part, float* out, hipStream_t s) {
-  const int nh = (dA_head || dD) ? d.H : 0;
+  const int nh = (dA_head || dD) ? d.H >> d.hs : 0;
   const int nr = out ? (width + 15) / 16 : 0;
   if (nh + nr == 0) return hipSuccess;
   hipLaunchKernelGGL(k_reduce_tail, dim3(nh + nr), dim3(1024), 0, s, d, b.chunks, b.dA_part, b.dD_part, dA_head, dD,

@@ -127,8 +127,10 @@ __global__ void __launch_bounds__(256) k_trapz_coef(SsdDims d, const int32_t* __
   int64_t start, end;
   const int seq = tz_seq(d, cu, row, start, end);
   float rho = 0.0f;
-  if (row + 1 < end) rho = to_f(beta[id + d.H]) * trapz_unfold(to_f(A[id + d.H]));
-  const float gm = to_f(gamma[id]);
+  const int Hr = d.H >> d.hs;  // the caller's heads
+  const int64_t ir = row * Hr + (h >> d.hs);
+  if (row + 1 < end) rho = to_f(beta[ir + Hr]) * trapz_unfold(to_f(A[ir + Hr]));
+  const float gm = to_f(gamma[ir]);
   b.tz_rho[id] = rho;
   b.tz_gam[id] = gm;
   b.tz_dt[id] = gm + rho;
@@ -159,7 +161,7 @@ __global__ void __launch_bounds__(256) k_trapz_coef_blk(SsdDims d, const T* __re
   const ChunkInfo ci = b.chunks[c];
   const int n = min(64, ci.len - 64 * kb);
   if (n <= 0) return;
-  const int H = d.H;
+  const int H = d.H, Hr = H >> d.hs;  // kernel heads, the caller's heads
   const int64_t r0 = (int64_t)ci.row0 + 64 * kb;
   // the sequence's end: the chunk table restarts chunks at every sequence start, so a chunk that ends
   // short of Q is its sequence's last; a full chunk is the last unless the next entry continues it
@@ -168,12 +170,12 @@ __global__ void __launch_bounds__(256) k_trapz_coef_blk(SsdDims d, const T* __re
   const int64_t end = (int64_t)ci.row0 + ci.len;  // rows of this chunk: [row0, end)
   for (int e = threadIdx.x; e < n * H; e += blockDim.x) {
     const int t = e / H, h = e - t * H;
-    const int64_t row = r0 + t, id = row * H + h;
+    const int64_t row = r0 + t, id = row * H + h, ir = row * Hr + (h >> d.hs);
     float rho = 0.0f;
     // the next token's beta folds into this one unless this is the sequence's last token
     if (row + 1 < end || (row + 1 == end && !seq_last_chunk))
-      rho = to_f(beta[id + H]) * trapz_unfold(to_f(A[id + H]));
-    const float gm = to_f(gamma[id]);
+      rho = to_f(beta[ir + Hr]) * trapz_unfold(to_f(A[ir + Hr]));
+    const float gm = to_f(gamma[ir]);
     b.tz_rho[id] = rho;
     b.tz_gam[id] = gm;
     b.tz_dt[id] = gm + rho;
@@ -232,20 +234,26 @@ __global__ void __launch_bounds__(256) k_trapz_grads(SsdDims d, const int32_t* _
                                                      const T* __restrict__ A, SsdBufs b, T* __restrict__ dgamma,
                                                      T* __restrict__ dbeta, T* __restrict__ dA) {
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= d.R * d.H) return;
-  const int64_t row = id / d.H;
-  const int h = (int)(id - row * d.H);
+  const int Hr = d.H >> d.hs;  // the caller's heads (tz_ddt, tz_da and the outputs are per caller head)
+  if (id >= d.R * Hr) return;
+  const int64_t row = id / Hr;
+  const int h = (int)(id - row * Hr) << d.hs;  // its first kernel head
   int64_t start, end;
   const int seq = tz_seq(d, cu, row, start, end);
   const bool inside = row < end;
-  if (dgamma)
-    dgamma[id] = from_f<T>(inside ? b.tz_ddt[id] + b.tz_cb[row * d.G + h / d.hpg] *
-                                                       b.xdy[tz_pos(d, b, row, start, seq) + (int64_t)h * d.Qpad]
-                                  : 0.0f);
+  if (dgamma) {
+    float xdy = 0.0f;
+    if (inside) {
+      const float* xd = b.xdy + tz_pos(d, b, row, start, seq) + (int64_t)h * d.Qpad;
+      xdy = xd[0];
+      if (d.hs) xdy += xd[d.Qpad];
+    }
+    dgamma[id] = from_f<T>(inside ? b.tz_ddt[id] + b.tz_cb[row * d.G + h / d.hpg] * xdy : 0.0f);
+  }
   float drho = 0.0f, rho = 0.0f;
   if (row > start && inside) {
-    drho = b.tz_ddt[id - d.H];
-    rho = b.tz_rho[id - d.H];
+    drho = b.tz_ddt[id - Hr];
+    rho = b.tz_rho[(row - 1) * d.H + h];
   }
   // (steep tokens: overwritten by k_trapz_dbeta_steep)
   if (dbeta) dbeta[id] = from_f<T>(drho * trapz_unfold(to_f(A[id])));
@@ -267,7 +275,9 @@ __global__ void __launch_bounds__(256) k_trapz_dbeta_steep(SsdDims d, const SsdB
                                                            const DS* __restrict__ dst, T* __restrict__ dbeta) {
   __shared__ float xs[SSD_MAX_HEADDIM], bs[SSD_MAX_DSTATE], csl[SSD_MAX_CHUNK], red[4];
   __shared__ unsigned char steep[SSD_MAX_CHUNK];
-  const int c = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  // (with two kernel heads per caller head, the block's head is the caller's and its terms sum over both)
+  const int c = blockIdx.x, hr = blockIdx.y, tid = threadIdx.x;
+  const int Hr = d.H >> d.hs, nk = 1 << d.hs, h = hr << d.hs;
   const ChunkInfo ci = b.chunks[c];
   const int len = min(ci.len, d.Q);
   if (len <= 0) return;
@@ -278,7 +288,7 @@ __global__ void __launch_bounds__(256) k_trapz_dbeta_steep(SsdDims d, const SsdB
   if (tid < len) {
     csl[tid] = cs[tid];
     // a sequence's first token has no beta input (x_prev = 0 there)
-    mine = !(ci.idx_in_seq == 0 && tid == 0) && to_f(A[(row0 + tid) * d.H + h]) < SSD_TRAPZ_STEEP;
+    mine = !(ci.idx_in_seq == 0 && tid == 0) && to_f(A[(row0 + tid) * Hr + hr]) < SSD_TRAPZ_STEEP;
     steep[tid] = mine ? 1 : 0;
   }
   if (!__syncthreads_or(mine)) return;
@@ -287,7 +297,8 @@ __global__ void __launch_bounds__(256) k_trapz_dbeta_steep(SsdDims d, const SsdB
   for (int i = 0; i < len; ++i) {
     if (!steep[i]) continue;  // block-uniform (LDS)
     const int64_t s = row0 + i - 1;
-    for (int p = tid; p < d.P; p += 256) xs[p] = to_f(x[(s * d.H + h) * d.P + p]);
+    const int PW = d.P << d.hs;  // the caller head's width: its kernel heads side by side
+    for (int p = tid; p < PW; p += 256) xs[p] = to_f(x[(s * d.H + h) * d.P + p]);
     for (int n = tid; n < d.N; n += 256) bs[n] = to_f(B[(s * d.G + g) * d.N + n]);
     __syncthreads();
     float acc = 0.0f;
@@ -297,20 +308,22 @@ __global__ void __launch_bounds__(256) k_trapz_dbeta_steep(SsdDims d, const SsdB
       const T* dyt = dy + (t * d.H + h) * d.P;
       float cb = 0.0f, xd = 0.0f;
       for (int n = 0; n < d.N; ++n) cb += to_f(ct[n]) * bs[n];
-      for (int p = 0; p < d.P; ++p) xd += xs[p] * to_f(dyt[p]);
+      for (int p = 0; p < PW; ++p) xd += xs[p] * to_f(dyt[p]);
       acc = exp_clamp(csl[tid] - csl[i]) * cb * xd;
     }
-    const DS* dsc = dst + ((int64_t)c * d.H + h) * d.Ppad * d.Npad;
     float sacc = 0.0f;
-    for (int e = tid; e < PN; e += 256) {
-      const int p = e / d.N, n = e - p * d.N;
-      sacc += xs[p] * bs[n] * to_f(dsc[p * d.Npad + n]);
+    for (int k = 0; k < nk; ++k) {
+      const DS* dsc = dst + ((int64_t)c * d.H + h + k) * d.Ppad * d.Npad;
+      for (int e = tid; e < PN; e += 256) {
+        const int p = e / d.N, n = e - p * d.N;
+        sacc += xs[k * d.P + p] * bs[n] * to_f(dsc[p * d.Npad + n]);
+      }
     }
     acc += exp_clamp(cs_last - csl[i]) * sacc;
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
     if ((tid & 63) == 0) red[tid >> 6] = acc;
     __syncthreads();
-    if (tid == 0) dbeta[(row0 + i) * d.H + h] = from_f<T>(red[0] + red[1] + red[2] + red[3]);
+    if (tid == 0) dbeta[(row0 + i) * Hr + hr] = from_f<T>(red[0] + red[1] + red[2] + red[3]);
     __syncthreads();  // xs, bs and red are reused by the next steep token
   }
 }
@@ -384,12 +397,12 @@ template <typename T>
 static hipError_t trapz_grads_t(const SsdDims& d, const SsdBufs& b, const void* A, const int32_t* cu, const void* x,
                                 const void* dy, const void* B, const void* C, void* dgamma, void* dbeta, void* dA,
                                 hipStream_t s) {
-  const int64_t n = d.R * d.H;
+  const int64_t n = d.R * (d.H >> d.hs);
   hipLaunchKernelGGL(k_trapz_grads<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d, cu,
                      reinterpret_cast<const T*>(A), b, reinterpret_cast<T*>(dgamma), reinterpret_cast<T*>(dbeta),
                      reinterpret_cast<T*>(dA));
   if (!dbeta) return hipGetLastError();
-  const dim3 grid((unsigned)d.max_chunks, (unsigned)d.H);
+  const dim3 grid((unsigned)d.max_chunks, (unsigned)(d.H >> d.hs));
   const T *tA = reinterpret_cast<const T*>(A), *tx = reinterpret_cast<const T*>(x),
           *tdy = reinterpret_cast<const T*>(dy), *tB = reinterpret_cast<const T*>(B),
           *tC = reinterpret_cast<const T*>(C);
