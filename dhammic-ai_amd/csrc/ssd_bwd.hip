@@ -1,22 +1,6 @@
-// Backward of the chunked SSD scan: dtype dispatch of the column / row
-// kernels (ssd_bwd_impl.h, instantiated in ssd_bwd_bf16.hip / ssd_bwd_f32.hip),
-// the finish kernel and the LDS sizes the host checks.
+// Backward of the chunked SSD scan: the finish kernel, and the LDS sizes of the column / row kernels
+// (ssd_bwd_impl.h), which bound the shapes the C ABI takes.
 #include "ssd_launch.h"
-
-hipError_t launch_bwd_col_bf16(const SsdDims&, const SsdBufs&, const SsdIn&, const void*, void*, void*, hipStream_t);
-hipError_t launch_bwd_col_f32(const SsdDims&, const SsdBufs&, const SsdIn&, const void*, void*, void*, hipStream_t);
-hipError_t launch_bwd_row_bf16(const SsdDims&, const SsdBufs&, const SsdIn&, const void*, void*, hipStream_t);
-hipError_t launch_bwd_row_f32(const SsdDims&, const SsdBufs&, const SsdIn&, const void*, void*, hipStream_t);
-
-hipError_t launch_bwd_col(int dtype, const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy,
-                          void* dx, void* dB, hipStream_t s) {
-  return dtype == 1 ? launch_bwd_col_bf16(d, b, in, dy, dx, dB, s) : launch_bwd_col_f32(d, b, in, dy, dx, dB, s);
-}
-
-hipError_t launch_bwd_row(int dtype, const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy,
-                          void* dC, hipStream_t s) {
-  return dtype == 1 ? launch_bwd_row_bf16(d, b, in, dy, dC, s) : launch_bwd_row_f32(d, b, in, dy, dC, s);
-}
 
 // ---------------------------------------------------------------------------
 // Finish: dcs per position, da = reverse in-chunk cumsum (the adjoint of the

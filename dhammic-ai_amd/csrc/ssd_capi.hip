@@ -28,13 +28,15 @@ struct Plan {
       o_tzcb, o_Dtok, o_hgam, o_hgamlo, o_dtrep, o_Drep, saved_bytes;
   size_t o_st, fwd_bytes;
   size_t o_dyp, o_dst, o_dtot, o_rowG, o_colG, o_eterm, o_dcs, o_xdx, o_dD, o_dA, o_dBp, o_dCp, o_dw, o_dS, o_dSf, o_dst16,
-      o_xdy, o_tzddt, o_tzda, bwd_bytes;
+      o_xdy, o_tzddt, o_tzda, o_bcb, o_fdS, bwd_bytes;
+  int f32_fbatch, f32_bbatch, f32_rhs, f32_rsl;  // fp32: units per batch (forward, backward), row slices
   int fused_bwd, nrowg;
   int rows_chunk;  // fused path: the chunk-resident row kernel (k_bwd_rows) instead of k_bwd_gemm
 };
 
-// `split`: whether a wide bf16 head may run as two heads of half its width (below).
-int plan(const ssd_desc_t* s, Plan* p, bool split = true) {
+// `tight`: the plan with the smallest forward workspaces (wide bf16 heads whole, fp32 S tiles in the chunk
+// states' place).
+int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
   if (!s || !p) return SSD_ERR_INVALID;
   memset(p, 0, sizeof(*p));
   if (s->batch < 1 || s->seqlen < 1 || s->nheads < 1 || s->headdim < 1 || s->ngroups < 1 || s->dstate < 1 ||
@@ -79,7 +81,7 @@ int plan(const ssd_desc_t* s, Plan* p, bool split = true) {
   // A, B, C and D, so a wider one whose half is a whole number of 16-byte vectors runs as two kernel heads of
   // P / 2 that share them: x, y, z, the states and their gradients keep their layout (heads are the slower
   // dimension), the cumsum launch repeats dt and D, and the finish sums the gradients of the pair.
-  if (split && s->dtype == SSD_DTYPE_BF16 && d.P > 64 && d.P % 16 == 0 && d.N % 8 == 0 && 2 * s->nheads <= kMaxGrid) {
+  if (!tight && s->dtype == SSD_DTYPE_BF16 && d.P > 64 && d.P % 16 == 0 && d.N % 8 == 0 && 2 * s->nheads <= kMaxGrid) {
     d.H *= 2;
     d.P /= 2;
     d.hs = 1;
@@ -111,6 +113,12 @@ int plan(const ssd_desc_t* s, Plan* p, bool split = true) {
     p->nrowg = bwd_main_num_sets(d);
     const int64_t per_slice = max_chunks * d.G * p->nrowg;
     ns = (256 + per_slice - 1) / per_slice;
+  } else if (s->dtype == SSD_DTYPE_F32) {
+    // four waves per SIMD in the column kernel (its waves are a unit's 32-token tiles; rowG in one partial per
+    // block of a unit)
+    p->nrowg = d.Qpad >= 192 ? 2 : 1;
+    const int64_t per_slice = max_chunks * d.G * (d.Qpad / 32);
+    ns = (4096 + per_slice - 1) / per_slice;
   } else {
     p->nrowg = 1;
     const int64_t per_slice = max_chunks * d.G * (d.Qpad / SSD_BLK);
@@ -130,6 +138,23 @@ int plan(const ssd_desc_t* s, Plan* p, bool split = true) {
                           lds_bwd_rows(d) <= kMaxLds
                       ? 1
                       : 0;
+  // the fp32 path: tiles of S and dS per unit (chunk, group), in batches that bound their memory, and the row
+  // kernel's head slices (up to two waves per SIMD over both roles, the tile term a slice of its own)
+  const int64_t units = max_chunks * d.G;
+  const bool f32 = s->dtype == SSD_DTYPE_F32;
+  const size_t unit_bytes = f32 ? f32_unit_floats(d) * sizeof(float) : 0;
+  if (f32) {
+    constexpr int64_t kFwdTiles = 512ll << 20, kBwdTiles = 1ll << 30;
+    const int64_t st_bytes = max_chunks * d.H * d.Ppad * d.Npad * 4;
+    const int64_t fb = (tight ? st_bytes : std::max(st_bytes, kFwdTiles)) / (int64_t)unit_bytes;
+    p->f32_fbatch = (int)std::max<int64_t>(1, std::min(units, fb));
+    p->f32_bbatch = (int)std::max<int64_t>(1, std::min(units, kBwdTiles / ((p->nslices + 1) * (int64_t)unit_bytes)));
+    int64_t nhs = 2048 / (units * 2 * (d.Qpad / 32)) - 1;
+    nhs = std::min<int64_t>(std::max<int64_t>(nhs, 1), d.hpg);
+    p->f32_rhs = (int)((d.hpg + nhs - 1) / nhs);
+    nhs = (d.hpg + p->f32_rhs - 1) / p->f32_rhs;
+    p->f32_rsl = nhs == 1 ? 1 : (int)nhs + 1;
+  }
   p->npass_blk = ((int64_t)d.Ppad * d.Npad + SSD_PASS_THREADS - 1) / SSD_PASS_THREADS;
   p->norm_blocks = R < 512 ? R : 512;
 
@@ -162,7 +187,8 @@ int plan(const ssd_desc_t* s, Plan* p, bool split = true) {
   p->o_Drep = (d.hs && d.has_D) ? take(H * sizeof(float)) : 0;
   p->saved_bytes = off;
   off = 0;
-  p->o_st = take(MC * H * PN * sizeof(float));
+  // (fp32: the scan's S tiles, once the chunk states have been used)
+  p->o_st = take(std::max(MC * H * PN * sizeof(float), p->f32_fbatch * unit_bytes));
   p->o_ffac = take(MC * H * d.Qpad * sizeof(float));
   p->o_ffac2 = d.trapz == SSD_TRAPZ_DROP_BETA_DA ? take(MC * H * d.Qpad * sizeof(float)) : 0;
   p->fwd_bytes = off;
@@ -178,9 +204,11 @@ int plan(const ssd_desc_t* s, Plan* p, bool split = true) {
   p->o_dD = take(MC * H * (d.Qpad / SSD_BLK) * sizeof(float));
   p->o_dA = take(MC * H * sizeof(float));
   const size_t bcn = (size_t)R * d.G * d.N * sizeof(float);
-  const bool parts = p->nslices > 1;
-  p->o_dBp = parts ? take(p->nslices * bcn) : 0;
-  p->o_dCp = parts ? take(p->nslices * bcn) : 0;
+  const int64_t nparts = f32 ? p->f32_rsl : p->nslices;
+  p->o_dBp = nparts > 1 ? take(nparts * bcn) : 0;
+  p->o_dCp = nparts > 1 ? take(nparts * bcn) : 0;
+  p->o_bcb = f32 ? take(p->f32_bbatch * unit_bytes) : 0;
+  p->o_fdS = f32 ? take(p->nslices * p->f32_bbatch * unit_bytes) : 0;
   const size_t nbq = (size_t)(d.Qpad / SSD_BLK);
   const bool tiles = p->fused_bwd;
   // one head slice: the tiles in bf16 (each is rounded to bf16 for the row kernel's products anyway)
@@ -240,9 +268,13 @@ void bind_bwd(const Plan& p, void* scratch, SsdBufs* b) {
   b->xdx = reinterpret_cast<float*>(s + p.o_xdx);
   b->dD_part = reinterpret_cast<float*>(s + p.o_dD);
   b->dA_part = reinterpret_cast<float*>(s + p.o_dA);
-  const bool parts = p.nslices > 1;
-  b->dB_part = parts ? reinterpret_cast<float*>(s + p.o_dBp) : nullptr;
-  b->dC_part = parts ? reinterpret_cast<float*>(s + p.o_dCp) : nullptr;
+  b->dB_part = p.o_dBp ? reinterpret_cast<float*>(s + p.o_dBp) : nullptr;
+  b->dC_part = p.o_dCp ? reinterpret_cast<float*>(s + p.o_dCp) : nullptr;
+  b->f32_cb = reinterpret_cast<float*>(s + p.o_bcb);
+  b->f32_dS = reinterpret_cast<float*>(s + p.o_fdS);
+  b->f32_batch = p.f32_bbatch;
+  b->f32_rhs = p.f32_rhs;
+  b->f32_rsl = p.f32_rsl;
   const bool tiles = p.fused_bwd;
   b->dS_tiles = (tiles && p.nslices > 1) ? reinterpret_cast<float*>(s + p.o_dS) : nullptr;
   b->dS_tiles16 = (tiles && p.nslices == 1) ? reinterpret_cast<bf16*>(s + p.o_dS) : nullptr;
@@ -309,6 +341,8 @@ int fwd_impl(Plan& p, const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* sav
   memset(&b, 0, sizeof(b));
   bind_saved(p, saved, &b);
   b.st = reinterpret_cast<float*>(scratch);
+  b.f32_cb = b.st;
+  b.f32_batch = p.f32_fbatch;
   b.fwd_fac = reinterpret_cast<float*>(static_cast<unsigned char*>(scratch) + p.o_ffac);
   b.fwd_fac2 = p.o_ffac2 ? reinterpret_cast<float*>(static_cast<unsigned char*>(scratch) + p.o_ffac2) : nullptr;
   // trapezoidal mode: the scan's dt is gamma + rho, written by the coefficient kernel; dt and D per kernel
@@ -362,8 +396,10 @@ int fwd_impl(Plan& p, const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* sav
     if (b.tz_cb_fwd) SSD_TRY(launch_trapz_dtok(d, b, Dk, s));
     SSD_TRY(launch_scan_fwd_chunk(d, b, in, yout, b.fast, s));
     SSD_TRY(tm.end(SSD_PH_FWD_SCAN));
-  } else
-    SSD_PHASE(tm, SSD_PH_FWD_SCAN, launch_chunk_scan_fwd(p.dtype, d, b, in, yout, s));
+  } else if (p.dtype == SSD_DTYPE_F32)
+    SSD_PHASE(tm, SSD_PH_FWD_SCAN, launch_f32_scan(d, b, in, yout, s));
+  else
+    SSD_PHASE(tm, SSD_PH_FWD_SCAN, launch_chunk_scan_fwd(d, b, in, yout, s));
   if (d.has_z) SSD_PHASE(tm, SSD_PH_NORM_FWD, launch_gated_norm_fwd(p.dtype, d, b, in, a->y, s));
   return SSD_OK;
 }
@@ -440,10 +476,10 @@ int ssd_fwd_noalloc(const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* strea
   Plan p;
   int st = plan(desc, &p);
   if (st != SSD_OK) return st;
-  // both forward workspaces, one after the other (the saved part is not kept for a backward); a wide head's
-  // pair takes a little more of it than the head itself, so near the limit the head runs whole
-  if (p.d.hs && align_up(p.saved_bytes) + p.fwd_bytes > (size_t)SSD_NOALLOC_SCRATCH_BYTES) {
-    st = plan(desc, &p, false);
+  // both forward workspaces, one after the other (the saved part is not kept for a backward); near the limit
+  // the plan with the smallest ones (a wide head's pair takes a little more than the head itself)
+  if (align_up(p.saved_bytes) + p.fwd_bytes > (size_t)SSD_NOALLOC_SCRATCH_BYTES) {
+    st = plan(desc, &p, true);
     if (st != SSD_OK) return st;
   }
   const size_t off = align_up(p.saved_bytes);
@@ -477,7 +513,7 @@ int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, 
   const bool fused = p.fused_bwd && d.vec_x && d.vec_bc;
   if (!fused) {
     b.ndcs = 1;
-    b.nrowg = 1;           // column / row kernels write one rowG partial
+    if (p.dtype != SSD_DTYPE_F32) b.nrowg = 1;  // the bf16 column / row kernels write one rowG partial
     b.dst16 = nullptr;     // and read dst in fp32
   }
   const bool fused_state = fused && state_fused_supported(p.dtype, d);
@@ -514,16 +550,32 @@ int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, 
       SSD_PHASE(t, SSD_PH_BWD_ROW,
                 bb.rows_chunk ? launch_bwd_rows(dd, bb, ii, dY, a->dB, a->dC, s)
                               : launch_bwd_gemm(dd, bb, ii, dY, a->dB, a->dC, s));
+    } else if (p.dtype == SSD_DTYPE_F32) {
+      // both sides per batch of units (one batch up to 1 GiB of tiles; past it the column phase's events
+      // bracket both)
+      const int units = dd.max_chunks * dd.G;
+      SSD_TRY(t.begin(SSD_PH_BWD_COL));
+      for (int u0 = 0; u0 < units; u0 += bb.f32_batch) {
+        const int n = std::min(bb.f32_batch, units - u0);
+        SSD_TRY(launch_f32_col(dd, bb, ii, dY, a->dx, u0, n, s));
+        if (u0 + n == units) {
+          SSD_TRY(t.end(SSD_PH_BWD_COL));
+          SSD_TRY(t.begin(SSD_PH_BWD_ROW));
+        }
+        SSD_TRY(launch_f32_row(dd, bb, ii, dY, a->dB, a->dC, u0, n, s));
+      }
+      SSD_TRY(t.end(SSD_PH_BWD_ROW));
     } else {
-      SSD_PHASE(t, SSD_PH_BWD_COL, launch_bwd_col(p.dtype, dd, bb, ii, dY, a->dx, a->dB, s));
-      SSD_PHASE(t, SSD_PH_BWD_ROW, launch_bwd_row(p.dtype, dd, bb, ii, dY, a->dC, s));
+      SSD_PHASE(t, SSD_PH_BWD_COL, launch_bwd_col(dd, bb, ii, dY, a->dx, a->dB, s));
+      SSD_PHASE(t, SSD_PH_BWD_ROW, launch_bwd_row(dd, bb, ii, dY, a->dC, s));
     }
     SSD_PHASE(t, SSD_PH_BWD_FINISH, launch_bwd_finish(p.dtype, dd, bb, ii, ddt, dA_tok, da32, s));
-    if (p.nslices > 1 && !fused) {
+    const int nparts = p.dtype == SSD_DTYPE_F32 ? p.f32_rsl : (fused ? 1 : (int)p.nslices);
+    if (nparts > 1) {
       const int64_t nelem = dd.R * dd.G * dd.N;
       SSD_TRY(t.begin(SSD_PH_BWD_REDUCE_BC));
-      SSD_TRY(launch_reduce_slices(p.dtype, nelem, (int)p.nslices, bb.dB_part, a->dB, s));
-      SSD_TRY(launch_reduce_slices(p.dtype, nelem, (int)p.nslices, bb.dC_part, a->dC, s));
+      SSD_TRY(launch_reduce_slices(p.dtype, nelem, nparts, bb.dB_part, a->dB, s));
+      SSD_TRY(launch_reduce_slices(p.dtype, nelem, nparts, bb.dC_part, a->dC, s));
       SSD_TRY(t.end(SSD_PH_BWD_REDUCE_BC));
     }
     return SSD_OK;

@@ -31,7 +31,7 @@ hipError_t launch_decay_chunk(int dtype, int batch, int H, int nch, int Q, const
 hipError_t launch_materialize_L(int dtype, int batch, int seqlen, int H, int Q, const void* a,
                                 void* L, hipStream_t s);
 
-// ssd_state.hip
+// ssd_state.hip (fp32: launch_chunk_state runs ssd_f32.hip's)
 // mode 0: st[c][h] = sum_l x_l^T (exp(cs_last - cs_l) dt_l B_l)      (forward chunk states)
 // mode 1: dst[c][h] = sum_l dy_l^T (exp(cs_l) C_l)                    (backward local dh)
 hipError_t launch_chunk_state(int dtype, int mode, const SsdDims& d, const SsdBufs& b,
@@ -67,16 +67,26 @@ hipError_t launch_scan_fwd_chunk(const SsdDims& d, const SsdBufs& b, const SsdIn
 size_t lds_scan_fwd_fact(const SsdDims& d);
 hipError_t launch_scan_fwd_fact(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s);
 
-// ssd_scan_fwd.hip
-hipError_t launch_chunk_scan_fwd(int dtype, const SsdDims& d, const SsdBufs& b, const SsdIn& in,
-                                 void* y, hipStream_t s);
+// ssd_scan_fwd.hip (bf16 shapes outside the fused path)
+hipError_t launch_chunk_scan_fwd(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s);
 size_t lds_chunk_scan_fwd(int dtype, const SsdDims& d);
 
+// ssd_f32.hip (fp32): the forward chunk scan, the chunk states (modes of launch_chunk_state), and the
+// backward of units [u0, u0 + n) (units: chunk * G + group), column side then row side
+size_t f32_unit_floats(const SsdDims& d);  // S (or dS) tiles of one unit
+hipError_t launch_f32_scan(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s);
+hipError_t launch_f32_state(int mode, const SsdDims& d, const SsdBufs& b, const void* U, const void* V, const float* dt,
+                            float* out, hipStream_t s);
+hipError_t launch_f32_col(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dx, int u0, int n,
+                          hipStream_t s);
+hipError_t launch_f32_row(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dB, void* dC, int u0,
+                          int n, hipStream_t s);
+
+// ssd_bwd_bf16.hip (bf16 shapes outside the fused path)
+hipError_t launch_bwd_col(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dx, void* dB,
+                          hipStream_t s);
+hipError_t launch_bwd_row(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dC, hipStream_t s);
 // ssd_bwd.hip
-hipError_t launch_bwd_col(int dtype, const SsdDims& d, const SsdBufs& b, const SsdIn& in,
-                          const void* dy, void* dx, void* dB, hipStream_t s);
-hipError_t launch_bwd_row(int dtype, const SsdDims& d, const SsdBufs& b, const SsdIn& in,
-                          const void* dy, void* dC, hipStream_t s);
 // ddt and da32 (fp32 per-token decay gradient, a_mode PER_TOKEN) are optional
 hipError_t launch_bwd_finish(int dtype, const SsdDims& d, const SsdBufs& b, const SsdIn& in,
                              float* ddt, void* dA_tok, float* da32, hipStream_t s);

@@ -93,6 +93,12 @@ struct SsdBufs {
   float* xdy;              // [max_chunks][H][Qpad] x_t . dy_t per head (the layout of xdx)
   float* tz_ddt;           // [R][H] gradient at dt = gamma + rho
   float* tz_da;            // [R][H] decay gradient of the scan (fp32)
+  // fp32 path (scratch), units (chunk, group) in batches of f32_batch: the S tiles, the dS tiles per head
+  // slice (ssd_f32.hip)
+  float* f32_cb;
+  float* f32_dS;
+  int f32_batch;
+  int f32_rhs, f32_rsl;    // the row kernel's heads per slice and its slices (the tile term's among them)
   int npass_blk, nslices, hslice, norm_blocks;
   int fused_bwd;           // 1: k_bwd_main + k_bwd_gemm (bf16), 0: column / row kernels
   int ndcs;                // dcs_off partials

@@ -1,5 +1,4 @@
-// Forward chunk scan kernel template (instantiated per dtype in
-// ssd_scan_fwd_bf16.hip / ssd_scan_fwd_f32.hip).
+// Forward chunk scan kernel template of the general bf16 path (instantiated in ssd_scan_fwd_bf16.hip).
 //   Y = (C B^T * L) X + exp(cs) C h_in^T (+ D x)
 #pragma once
 

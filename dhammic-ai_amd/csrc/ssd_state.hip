@@ -87,19 +87,13 @@ static size_t lds_chunk_state(int dtype, const SsdDims& d) {
 
 hipError_t launch_chunk_state(int dtype, int mode, const SsdDims& d, const SsdBufs& b, const void* U,
                               const void* V, const float* dt, float* out, hipStream_t s) {
+  if (dtype != 1) return launch_f32_state(mode, d, b, U, V, dt, out, s);
   dim3 grid(d.max_chunks, d.H);
   const size_t lds = lds_chunk_state(dtype, d);
-  if (dtype == 1) {
-    auto k = mode == 0 ? k_chunk_state<bf16, 0> : k_chunk_state<bf16, 1>;
-    ensure_lds(k, lds);
-    hipLaunchKernelGGL(k, grid, dim3(256), lds, s, d, b.chunks, b.cs, reinterpret_cast<const bf16*>(U),
-                       reinterpret_cast<const bf16*>(V), dt, out);
-  } else {
-    auto k = mode == 0 ? k_chunk_state<float, 0> : k_chunk_state<float, 1>;
-    ensure_lds(k, lds);
-    hipLaunchKernelGGL(k, grid, dim3(256), lds, s, d, b.chunks, b.cs, reinterpret_cast<const float*>(U),
-                       reinterpret_cast<const float*>(V), dt, out);
-  }
+  auto k = mode == 0 ? k_chunk_state<bf16, 0> : k_chunk_state<bf16, 1>;
+  ensure_lds(k, lds);
+  hipLaunchKernelGGL(k, grid, dim3(256), lds, s, d, b.chunks, b.cs, reinterpret_cast<const bf16*>(U),
+                     reinterpret_cast<const bf16*>(V), dt, out);
   return hipGetLastError();
 }
 
