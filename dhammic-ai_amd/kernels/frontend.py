@@ -28,7 +28,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from . import _capi as C_
-from .ssd_scan import _code, _p, _stream
+from .ssd_scan import _code, _on, _p, _stream
 
 __all__ = ["fused_trapezoidal", "FusedTrapezoidal", "fused_rope", "FusedRoPE", "fused_inproj_split",
            "FusedInProjSplit", "FusedInProjSplitModule"]
@@ -57,7 +57,7 @@ class FusedTrapezoidal(torch.autograd.Function):
         outs = [torch.empty_like(x) for _ in range(4)]
         lib = C_.load()
         dev = x.device
-        with torch.cuda.device(dev):
+        with _on(dev):
             st = lib.ssd_trapezoidal_fwd(code, rows, H, _p(x), _p(lam), _p(bias), _p(alog), *[_p(o) for o in outs],
                                          _stream(dev))
         C_.check(st, "ssd_trapezoidal_fwd")
@@ -78,7 +78,7 @@ class FusedTrapezoidal(torch.autograd.Function):
         d_alog = torch.empty(H, dtype=torch.float32, device=x.device)
         lib = C_.load()
         ws = torch.empty(lib.ssd_trapezoidal_bwd_workspace(rows, H), dtype=torch.uint8, device=x.device)
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             st = lib.ssd_trapezoidal_bwd(_code(dtype, "dt_raw"), rows, H, _p(x), _p(lam), _p(bias), _p(alog),
                                          *[_p(g) for g in gs], _p(d_x), _p(d_lam), _p(d_bias), _p(d_alog), _p(ws),
                                          ws.numel(), _stream(x.device))
@@ -109,7 +109,7 @@ class FusedRoPE(torch.autograd.Function):
         xc, ac = x.contiguous(), angles.contiguous()
         out = torch.empty_like(xc)
         lib = C_.load()
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             st = lib.ssd_rope_fwd(_code(x.dtype, "x"), _code(angles.dtype, "angles"), B, T, H, half, int(aH == H),
                                   _p(xc), _p(ac), _p(out), _stream(x.device))
         C_.check(st, "ssd_rope_fwd")
@@ -124,7 +124,7 @@ class FusedRoPE(torch.autograd.Function):
         dx = torch.empty_like(xc)
         dang = torch.empty_like(ac)
         lib = C_.load()
-        with torch.cuda.device(xc.device):
+        with _on(xc.device):
             st = lib.ssd_rope_bwd(_code(xc.dtype, "x"), _code(ac.dtype, "angles"), B, T, H, D // 2,
                                   int(ac.shape[2] == H), _p(xc), _p(ac), _p(dyc), _p(dx), _p(dang),
                                   _stream(xc.device))

@@ -25,7 +25,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from . import _capi as C_
-from .ssd_scan import _p, _stream
+from .ssd_scan import _on, _p, _stream
 
 __all__ = ["fused_lmhead_xent", "FusedLMHeadXent", "FusedLMHeadXentModule", "ChunkedLMHeadXent"]
 
@@ -92,7 +92,7 @@ class FusedLMHeadXent(torch.autograd.Function):
         mask = torch.empty(M, dtype=torch.int32, device=dev)
         lib = C_.load()
         ws = torch.empty(lib.ssd_lmhead_xent_workspace(M, V), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             st = lib.ssd_lmhead_xent_fwd(M, V, D, _p(hk), _p(wk), _p(t), int(ignore_index), _p(logZ), _p(tl),
                                          _p(mask), _p(ws), ws.numel(), _stream(dev))
         C_.check(st, "ssd_lmhead_xent_fwd")
@@ -128,7 +128,7 @@ class FusedLMHeadXent(torch.autograd.Function):
         lib = C_.load()
         for r0 in range(0, M, rows):
             n = min(rows, M - r0)
-            with torch.cuda.device(dev):
+            with _on(dev):
                 st = lib.ssd_lmhead_xent_dlogits(M, V, D, r0, n, _p(h), _p(w), _p(t), ctx.ignore_index, _p(logZ),
                                                  _p(scale), _p(G), ldg, _stream(dev))
             C_.check(st, "ssd_lmhead_xent_dlogits")
@@ -161,7 +161,7 @@ class FusedLMHeadXent(torch.autograd.Function):
         lib = C_.load()
         for r0 in range(0, M, rows):
             n = min(rows, M - r0)
-            with torch.cuda.device(dev):
+            with _on(dev):
                 st = lib.ssd_lmhead_xent_dlogits_split(M, V, hk.shape[1], r0, n, _p(hk), _p(wk), _p(t),
                                                        ctx.ignore_index, _p(logZ), _p(scale), _p(G), _p(G_lo), ldg,
                                                        _stream(dev))

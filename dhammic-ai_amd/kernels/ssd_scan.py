@@ -27,10 +27,12 @@ first access (they are never needed by the kernels).
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import functools
 import weakref
-import dataclasses
 from dataclasses import dataclass
+from typing import NamedTuple
 
 import torch
 
@@ -48,15 +50,24 @@ def _code(dtype, what):
 
 
 def _p(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """The tensor's address as ctypes takes it (an int, or None)."""
+    return None if t is None else t.data_ptr()
 
 
 def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    """The current stream's handle on dev (torch.cuda.current_stream builds a Stream object, 3 us a call)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if dev.index is None else dev.index)
 
 
-@dataclass(frozen=True)
-class _Cfg:
+_HERE = contextlib.nullcontext()
+
+
+def _on(dev):
+    """A context with dev current: nothing to do where it already is (torch.cuda.device costs 5 us a call)."""
+    return _HERE if dev.index is None or dev.index == torch.cuda.current_device() else torch.cuda.device(dev)
+
+
+class _Cfg(NamedTuple):
     chunk: int
     a_mode: int
     nseq: int
@@ -69,17 +80,21 @@ class _Cfg:
 
 
 def _desc(cfg: _Cfg, x, B, dt, D, z, init, has_dfinal=False):
-    b, T, H, P = x.shape
+    return _desc_of(cfg, x.shape, B.shape[2], B.shape[3], x.dtype, dt is not None, D is not None, z is not None,
+                    init is not None, has_dfinal)
+
+
+def _desc_of(cfg: _Cfg, x_shape, G, N, dtype, has_dt, has_D, has_z, has_init, has_dfinal):
     d = C_.SsdDesc()
-    d.batch, d.seqlen, d.nheads, d.headdim = b, T, H, P
-    d.ngroups, d.dstate, d.chunk, d.nseq = B.shape[2], B.shape[3], cfg.chunk, cfg.nseq
-    d.dtype = _code(x.dtype, "x")
+    d.batch, d.seqlen, d.nheads, d.headdim = x_shape
+    d.ngroups, d.dstate, d.chunk, d.nseq = G, N, cfg.chunk, cfg.nseq
+    d.dtype = _code(dtype, "x")
     d.state_dtype = cfg.state_code
     d.a_mode = cfg.a_mode
-    d.has_dt = int(dt is not None)
-    d.has_D = int(D is not None)
-    d.has_z = int(z is not None)
-    d.has_init = int(init is not None)
+    d.has_dt = int(has_dt)
+    d.has_D = int(has_D)
+    d.has_z = int(has_z)
+    d.has_init = int(has_init)
     d.has_dfinal = int(has_dfinal)
     d.varlen = int(cfg.varlen)
     d.want_final = int(not cfg.trapz)
@@ -104,8 +119,11 @@ def _head_split(lib, cfg: _Cfg, x, B, dt, D, z, init):
     and their gradients keep their memory layout (heads are the slower dimension), B and C their
     groups (each of the k heads of a group's head reads the same group), and dt, A, D and the
     trapezoidal coefficients are repeated per head, their gradients summed back."""
-    b, T, H, P = x.shape
-    desc = _desc(cfg, x, B, dt, D, z, init)
+    return _split_factor(lib, _desc(cfg, x, B, dt, D, z, init))
+
+
+def _split_factor(lib, desc):
+    H, P = desc.nheads, desc.headdim
     first = lib.ssd_validate(ctypes.byref(desc))
     if first != C_.SSD_ERR_UNSUPPORTED:
         return 1
@@ -119,6 +137,36 @@ def _head_split(lib, cfg: _Cfg, x, B, dt, D, z, init):
         if st != C_.SSD_ERR_UNSUPPORTED:
             break
     return 1  # (the caller's own validation then reports the limit)
+
+
+class _Plan(NamedTuple):
+    """What one shape of call needs from the host: the heads' split (``_head_split``), the descriptor the library
+    reads, and the bytes of its workspaces."""
+    k: int
+    desc: object   # ctypes.byref(SsdDesc), only read once made
+    saved: int
+    fwd: int
+    bwd: int
+
+
+@functools.lru_cache(maxsize=512)
+def _plan(cfg: _Cfg, x_shape, G, N, dtype, has_dt, has_D, has_z, has_init, has_dfinal):
+    """The plan by the sizes and options alone (no tensor, address or device enters it), so that a training loop's
+    calls find it made; errors are raised anew each time. Building it took 15 of a call's 60 us on the host."""
+    lib = C_.load()
+    args = (G, N, dtype, has_dt, has_D, has_z, has_init, has_dfinal)
+    k = _split_factor(lib, _desc_of(cfg, x_shape, *args))
+    b, T, H, P = x_shape
+    desc = _desc_of(cfg, (b, T, H * k, P // k), *args)
+    ref = ctypes.byref(desc)
+    C_.check(lib.ssd_validate(ref), "ssd_fwd")
+    return _Plan(k, ref, *(lib.ssd_workspace_bytes(ref, w)
+                           for w in (C_.SSD_WS_SAVED, C_.SSD_WS_FWD_SCRATCH, C_.SSD_WS_BWD_SCRATCH)))
+
+
+def _plan_for(cfg, x, B, dt, D, z, init, has_dfinal=False):
+    return _plan(cfg, tuple(x.shape), B.shape[2], B.shape[3], x.dtype, dt is not None, D is not None, z is not None,
+                 init is not None, has_dfinal)
 
 
 def _split_heads(k, cfg: _Cfg, x, dt, A, D, z, init, gamma, beta):
@@ -171,10 +219,10 @@ def _forward(cfg: _Cfg, x, dt, A, B, C, D, z, w, init, cu, events=None, gamma=No
     lib = C_.load()
     _check_device(x, dt, A, B, C, D, z, w, init, cu, gamma, beta)
     b, T, H0, P0 = x.shape
-    k = _head_split(lib, cfg, x, B, dt, D, z, init)
-    x, dt, A, D, z, init, gamma, beta = _split_heads(k, cfg, x, dt, A, D, z, init, gamma, beta)
-    desc = _desc(cfg, x, B, dt, D, z, init)
-    C_.check(lib.ssd_validate(ctypes.byref(desc)), "ssd_fwd")
+    plan = _plan_for(cfg, x, B, dt, D, z, init)
+    k = plan.k
+    if k > 1:
+        x, dt, A, D, z, init, gamma, beta = _split_heads(k, cfg, x, dt, A, D, z, init, gamma, beta)
     b, T, H, P = x.shape
     N = B.shape[3]
     dev = x.device
@@ -183,16 +231,13 @@ def _forward(cfg: _Cfg, x, dt, A, B, C, D, z, w, init, cu, events=None, gamma=No
     final = None if cfg.trapz else torch.empty((cfg.nseq, H, P, N), dtype=sdt, device=dev)
     acs = (torch.empty((b, H, T // cfg.chunk, cfg.chunk), dtype=x.dtype, device=dev)
            if cfg.want_acs else x.new_empty(0))
-    saved = torch.empty(lib.ssd_workspace_bytes(ctypes.byref(desc), C_.SSD_WS_SAVED), dtype=torch.uint8,
-                        device=dev)
-    scratch = torch.empty(lib.ssd_workspace_bytes(ctypes.byref(desc), C_.SSD_WS_FWD_SCRATCH),
-                          dtype=torch.uint8, device=dev)
+    saved = torch.empty(plan.saved, dtype=torch.uint8, device=dev)
+    scratch = torch.empty(plan.fwd, dtype=torch.uint8, device=dev)
     args = C_.SsdFwdArgs(_p(x), _p(dt), _p(A), _p(B), _p(C), _p(D), _p(z), _p(w), _p(init), _p(cu),
                          _p(y), _p(final), _p(acs) if cfg.want_acs else None,
                          None if events is None else ctypes.cast(events, ctypes.c_void_p), _p(gamma), _p(beta))
-    with torch.cuda.device(dev):
-        st = lib.ssd_fwd(ctypes.byref(desc), ctypes.byref(args), _p(saved), saved.numel(), _p(scratch),
-                         scratch.numel(), _stream(dev))
+    with _on(dev):
+        st = lib.ssd_fwd(plan.desc, ctypes.byref(args), _p(saved), plan.saved, _p(scratch), plan.fwd, _stream(dev))
     C_.check(st, "ssd_fwd")
     if k > 1:  # back to the caller's heads (the k copies of a head's cumsum are equal)
         y = y.view(b, T, H0, P0)
@@ -219,9 +264,10 @@ def _backward(cfg: _Cfg, saved_ws, x, dt, A, B, C, D, z, w, init, cu, dy, dfinal
     ``A`` is the decay input the forward took (A_cumsum with a cache)."""
     lib = C_.load()
     b, T, H0, P0 = x.shape
-    k = _head_split(lib, cfg, x, B, dt, D, z, init)
-    x, dt, A, D, z, init, gamma, beta = _split_heads(k, cfg, x, dt, A, D, z, init, gamma, beta)
-    desc = _desc(cfg, x, B, dt, D, z, init, has_dfinal=dfinal is not None)
+    plan = _plan_for(cfg, x, B, dt, D, z, init, dfinal is not None)
+    k = plan.k
+    if k > 1:
+        x, dt, A, D, z, init, gamma, beta = _split_heads(k, cfg, x, dt, A, D, z, init, gamma, beta)
     dev = x.device
     dy = torch.zeros_like(x) if dy is None else dy.contiguous().view(x.shape)
     if dy.dtype != x.dtype:
@@ -240,17 +286,16 @@ def _backward(cfg: _Cfg, saved_ws, x, dt, A, B, C, D, z, w, init, cu, dy, dfinal
         "gamma": torch.empty_like(gamma) if gamma is not None else None,
         "beta": torch.empty_like(beta) if beta is not None else None,
     }
-    scratch = torch.empty(lib.ssd_workspace_bytes(ctypes.byref(desc), C_.SSD_WS_BWD_SCRATCH),
-                          dtype=torch.uint8, device=dev)
+    scratch = torch.empty(plan.bwd, dtype=torch.uint8, device=dev)
     args = C_.SsdBwdArgs(_p(x), _p(dt), _p(A), _p(B), _p(C), _p(D), _p(z), _p(w), _p(init), _p(cu),
                          _p(dy), _p(dfinal),
                          _p(g["x"]), _p(g["dt"]), _p(g["A"]), _p(g["B"]), _p(g["C"]), _p(g["D"]),
                          _p(g["z"]), _p(g["w"]), _p(g["init"]),
                          None if events is None else ctypes.cast(events, ctypes.c_void_p),
                          _p(gamma), _p(beta), _p(g["gamma"]), _p(g["beta"]))
-    with torch.cuda.device(dev):
-        st = lib.ssd_bwd(ctypes.byref(desc), ctypes.byref(args), _p(saved_ws), saved_ws.numel(), _p(scratch),
-                         scratch.numel(), _stream(dev))
+    with _on(dev):
+        st = lib.ssd_bwd(plan.desc, ctypes.byref(args), _p(saved_ws), saved_ws.numel(), _p(scratch), plan.bwd,
+                         _stream(dev))
     C_.check(st, "ssd_bwd")
     if k > 1:  # back to the caller's heads: views of the split ones, or sums over each head's k copies
         a_dim = {C_.SSD_A_PER_HEAD: 0, C_.SSD_A_PER_TOKEN: -1}.get(cfg.a_mode, -1)
@@ -336,7 +381,7 @@ class _LazyCache(dict):
             b, H, nch, Q = acs.shape
             desc = _cache_desc(self._a, self._chunk)
             dev = acs.device
-            with torch.cuda.device(dev):
+            with _on(dev):
                 if key == "L":
                     v = torch.empty((b, H, nch, Q, Q), dtype=acs.dtype, device=dev)
                     C_.check(lib.ssd_materialize_L(ctypes.byref(desc), _p(self._a), _p(v), _stream(dev)),
@@ -536,7 +581,7 @@ def _rechunk_plan(plan, chunk):
         a32 = acs.float().view(b, H, nch, Q // qk, qk)
         base = torch.cat([torch.zeros_like(a32[..., :1, -1:]), a32[..., :-1, -1:]], dim=-2)
         acs = (a32 - base).reshape(b, H, nch * (Q // qk), qk).to(acs.dtype).contiguous()
-    return _CachePlan(dataclasses.replace(plan.cfg, chunk=qk, want_acs=False), acs, plan.A_used)
+    return _CachePlan(plan.cfg._replace(chunk=qk, want_acs=False), acs, plan.A_used)
 
 
 def _chunk_cumsum(a, chunk):
