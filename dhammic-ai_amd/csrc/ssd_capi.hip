@@ -32,6 +32,7 @@ struct Plan {
   int f32_fbatch, f32_bbatch, f32_rhs, f32_rsl;  // fp32: units per batch (forward, backward), row slices
   int fused_bwd, nrowg;
   int rows_chunk;  // fused path: the chunk-resident row kernel (k_bwd_rows) instead of k_bwd_gemm
+  int head_bwd;    // fused path, one head per group: k_bwd_head in place of the column and row kernels
 };
 
 // `tight`: the plan with the smallest forward workspaces (wide bf16 heads whole, fp32 S tiles in the chunk
@@ -155,6 +156,8 @@ int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
     nhs = (d.hpg + p->f32_rhs - 1) / p->f32_rhs;
     p->f32_rsl = nhs == 1 ? 1 : (int)nhs + 1;
   }
+  p->head_bwd = p->fused_bwd && !force_block && !force_chunk && bwd_head_supported(p->dtype, d) &&
+                lds_bwd_head(d) <= kMaxLds && max_chunks * d.H <= INT32_MAX;
   p->npass_blk = ((int64_t)d.Ppad * d.Npad + SSD_PASS_THREADS - 1) / SSD_PASS_THREADS;
   p->norm_blocks = R < 512 ? R : 512;
 
@@ -516,6 +519,8 @@ int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, 
     if (p.dtype != SSD_DTYPE_F32) b.nrowg = 1;  // the bf16 column / row kernels write one rowG partial
     b.dst16 = nullptr;     // and read dst in fp32
   }
+  const bool head = fused && p.head_bwd;
+  if (head) b.nrowg = b.ndcs = 1;  // (its row sums of G and its decay term are whole)
   const bool fused_state = fused && state_fused_supported(p.dtype, d);
   if (fused_state) b.npass_blk = state_fused_slices(d);  // dtot partials: one per 32 x 32 state tile
   const void* dY = a->dy;
@@ -540,7 +545,9 @@ int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, 
                                         dd.has_init ? a->dinit : nullptr, s));
       }
     }
-    if (fused) {
+    if (head) {
+      SSD_PHASE(t, SSD_PH_BWD_COL, launch_bwd_head(dd, bb, ii, dY, a->dx, a->dB, a->dC, s));
+    } else if (fused) {
       // factorised column kernel, then the exact one on the (chunk, head) pairs it cannot take;
       // the row phase builds dB / dC
       SSD_TRY(t.begin(SSD_PH_BWD_COL));
@@ -611,15 +618,19 @@ int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, 
       SSD_PHASE(tm, SSD_PH_BWD_STATE, launch_chunk_state(p.dtype, 1, dm, bw, dY, a->C, in.dt, bw.dst, s));
       SSD_PHASE(tm, SSD_PH_BWD_PASS, launch_state_pass_bwd(p.dtype, p.state_dtype, dm, bw, nullptr, nullptr, s));
     }
-    SSD_TRY(tm.begin(SSD_PH_BWD_COL));
-    SSD_TRY(launch_bwd_fact(dm, b, in, dY, a->dx, s));
-    SSD_TRY(launch_bwd_main(dm, b, in, dY, a->dx, true, s));
-    SSD_TRY(tm.end(SSD_PH_BWD_COL));
-    if (b.rows_chunk) {
-      // the chunk-resident row kernel takes the decay term over hgam in the same blocks
-      SsdBufs br = b;
-      br.hdec = b.hgam;
-      br.hdec_lo = b.hgam_lo;
+    SsdBufs br = b;  // the decay term over hgam in the same blocks (head kernel, chunk-resident row kernel)
+    br.hdec = b.hgam;
+    br.hdec_lo = b.hgam_lo;
+    if (head) {
+      SSD_PHASE(tm, SSD_PH_BWD_COL, launch_bwd_head(dm, br, in, dY, a->dx, a->dB, a->dC, s));
+    } else {
+      SSD_TRY(tm.begin(SSD_PH_BWD_COL));
+      SSD_TRY(launch_bwd_fact(dm, b, in, dY, a->dx, s));
+      SSD_TRY(launch_bwd_main(dm, b, in, dY, a->dx, true, s));
+      SSD_TRY(tm.end(SSD_PH_BWD_COL));
+    }
+    if (head) {
+    } else if (b.rows_chunk) {
       SSD_PHASE(tm, SSD_PH_BWD_ROW, launch_bwd_rows(dm, br, in, dY, a->dB, a->dC, s));
     } else {
       SSD_PHASE(tm, SSD_PH_BWD_ROW, launch_bwd_gemm(dm, b, in, dY, a->dB, a->dC, s));

@@ -105,6 +105,14 @@ int bwd_main_num_sets(const SsdDims& d);
 hipError_t launch_bwd_main(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dx, bool fixup,
                            hipStream_t s);
 
+// ssd_bwd_head.hip (fused path, one head per group): the whole of a (chunk, head)'s backward but the walks and the
+// finish: dx, dB, dC, the decay gradient's terms (one rowG and one dcs_off partial), exact decays (no fixup).
+// b.hdec / b.hdec_lo: the decay term's states with d.gdec
+bool bwd_head_supported(int dtype, const SsdDims& d);
+size_t lds_bwd_head(const SsdDims& d);
+hipError_t launch_bwd_head(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dx, void* dB,
+                           void* dC, hipStream_t s);
+
 // ssd_bwd_fact.hip (same shapes and grid as k_bwd_main): the factorised-decay column kernel
 size_t lds_bwd_fact(const SsdDims& d);
 hipError_t launch_bwd_fact(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dx,
