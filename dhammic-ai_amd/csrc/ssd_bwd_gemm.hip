@@ -26,6 +26,11 @@
 // whose issue waits for room in the texture unit's queue. LDS rows are unpadded; 16-byte granules are
 // permuted per row so that transposed reads (h_in, dst) and row reads (x, dy)
 // hit distinct banks.
+//
+// Few blocks (a short batch of one or two groups): the walk over the heads is a serial chain of ~2.2 us each and the
+// tile terms another one (each step sums the column slices' dS partials, eight in flight: 70 -> 58 us for 24 heads of
+// one 256-token chunk), so both go to slices with fp32 partials of dB / dC (58 -> 22 us with the launch that sums
+// them; gemm_slices in ssd_capi.hip has the rule).
 #include "ssd_launch.h"
 #include "ssd_tile.h"
 
@@ -60,7 +65,9 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
                                                   const float* __restrict__ dS_fix, const int32_t* __restrict__ fast,
                                                   float* __restrict__ dcs_off, bf16* __restrict__ dB,
                                                   bf16* __restrict__ dC, const float* __restrict__ tz_gam,
-                                                  float* __restrict__ xdy) {
+                                                  float* __restrict__ xdy, int hslice, int tsteps,
+                                                  float* __restrict__ dB_part,
+                                                  float* __restrict__ dC_part) {
   using Cfg = GemmCfg<PT, NT>;
   constexpr int PP = Cfg::PP, NP = Cfg::NP, NTW = (NT + 1) / 2, NK = PP / 16;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -85,7 +92,11 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
   const int nrows = min(64, ci.len - 64 * kb);
   const int64_t brow = (int64_t)d.G * d.N, xrow = (int64_t)d.H * d.P;
   const int MC = d.max_chunks, Qpad = d.Qpad;
-  const int h0 = g * d.hpg, h1 = h0 + d.hpg;
+  // this block's heads: all of the group's, then the tile terms; or (dB_part set) slice z of hslice heads, with more
+  // slices for tsteps steps of the tile terms each
+  const bool sliced = dB_part != nullptr;
+  const int hz = blockIdx.z * hslice, nhd = max(0, min(hslice, d.hpg - hz));
+  const int h0 = g * d.hpg + hz;
 
   // ---- one head's inputs into a ring slot (kPerWave DMA instructions per issuing wave) ----
   // Issuing waves 0-1 (waves 4-5) load h_in and the x rows, 2-3 dst and the dy rows, each its own fixed
@@ -218,13 +229,13 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
   // head order rotated per chunk (the blocks of one chunk keep the same order, so they still share each
   // head's tiles through L2): the resident blocks then read different 128-byte columns of the 8 KB token
   // rows at any moment instead of all the same one (HBM channel spread)
-  const int nhd = h1 - h0, hrot = c % nhd;
+  const int hrot = nhd ? c % nhd : 0;
   auto head = [&](int k) { const int m = k + hrot; return h0 + (m >= nhd ? m - nhd : m); };
   if (brole) {
-    issue(head(0), smem);
+    if (0 < nhd) issue(head(0), smem);
     if (1 < nhd) issue(head(1), smem + Cfg::kSlot);
   }
-  if (use_lo) load_lo(head(0));
+  if (use_lo && 0 < nhd) load_lo(head(0));
   // head k reads slot k % 3 and refills slot (k + 2) % 3; the loop below is unrolled over the three
   // slots, so every slot address is a constant
   auto head_step = [&](int k, const unsigned char* __restrict__ cur, unsigned char* __restrict__ nxt) {
@@ -307,6 +318,34 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
   }
 
   if (d.da_only) return;  // decay gradient only: the Y_off term above is all it needs
+  // dC (dC waves) / dB rows t: bf16, or a slice's partial sums
+  auto put = [&]() {
+    if (!tok) return;
+    const int64_t row = (int64_t)(ci.row0 + t) * brow + (int64_t)g * d.N;
+    float* part = sliced ? (brole ? dB_part : dC_part) + (int64_t)blockIdx.z * d.R * brow + row : nullptr;
+    bf16* out = (brole ? dB : dC) + row;
+#pragma unroll
+    for (int q = 0; q < NTW; ++q) {
+      const int nt = nh * NTW + q;
+      if (nt >= NT) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n0 = 32 * nt + 8 * r + 4 * hh;
+        if (n0 >= d.N) continue;
+        if (sliced) {
+          floatx4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = acc[q][4 * r + e];
+          *reinterpret_cast<floatx4*>(part + n0) = o;
+        } else {
+          bf16x4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = (bf16)acc[q][4 * r + e];
+          *reinterpret_cast<bf16x4*>(out + n0) = o;
+        }
+      }
+    }
+  };
   // ---- tile terms, both roles at once: step m of the dC waves takes tile (kb, m), m <= kb, with the B
   // rows of block m (dC += dS B); step m of the dB waves tile (kb + m, kb), kb + m < nbl, with the C rows
   // of block kb + m (dB += dS^T C). Each role has its LDS buffer pair; every thread stages one 8-element
@@ -323,12 +362,34 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
     __syncthreads();  // the ring's last reads are done
     if (!brole && nh == 0 && hh == 0) s_dcb[t_loc] = dcb;
   }
+  if (sliced && nhd > 0) {
+    if (d.trapz) {  // the slice's part of dS's diagonal: dC_t += dcb B_t, dB_t += dcb C_t
+      __syncthreads();
+      const float dg = s_dcb[t_loc];
+      const __amdgpu_buffer_rsrc_t rg = buf_rsrc((brole ? Cm : Bm) + (int64_t)ci.row0 * brow + (int64_t)g * d.N);
+#pragma unroll
+      for (int q = 0; q < NTW; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int n0 = 32 * (nh * NTW + q) + 8 * r + 4 * hh;
+          const bool ok = tok && n0 < d.N;
+          const bf16x4 v = __builtin_bit_cast(bf16x4, __builtin_amdgcn_raw_buffer_load_b64(
+              rg, ok ? (int)(t * brow + n0) * 2 : SSD_BUF_SIZE, 0, 0));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[q][4 * r + e] = fmaf(dg, (float)v[e], acc[q][4 * r + e]);
+        }
+    }
+    put();
+    return;
+  }
   // heads of the group the factorised kernel left to the exact fixup: their dS is in dS_fix
   bool slow = false;
   if (fast)
-    for (int hq = h0 + (int)threadIdx.x; hq < h1; hq += 512) slow = slow || fast[(int64_t)c * d.H + hq] == 0;
+    for (int hq = g * d.hpg + (int)threadIdx.x; hq < (g + 1) * d.hpg; hq += 512) slow = slow || fast[(int64_t)c * d.H + hq] == 0;
   const bool any_fix = __syncthreads_or(slow);
-  fetch(0);
+  const int st0 = sliced ? (blockIdx.z - (d.hpg + hslice - 1) / hslice) * tsteps : 0;
+  const int st1 = sliced ? min(nsteps, st0 + tsteps) : nsteps;
+  if (st0 < st1) fetch(st0);
   // one tile's piece: the fetched bf16 values, or the fp32 slice partials summed here; plus the fixup
   // heads' dS and (trapezoidal mode, tile (kb, kb)) the diagonal sum_h gamma (x_t . dy_t)
   auto store_piece = [&](bf16* tS, int ti, int tj, const bf16x8& pre) {
@@ -340,9 +401,20 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
       const float* src = dS + tile0 + ((int64_t)ti * nb + tj) * 4096 + pr * 64 + pk;
       floatx4 s0 = *reinterpret_cast<const floatx4*>(src);
       floatx4 s1 = *reinterpret_cast<const floatx4*>(src + 4);
-      for (int sl = 1; sl < nslices; ++sl) {
-        s0 += *reinterpret_cast<const floatx4*>(src + sl * sstride);
-        s1 += *reinterpret_cast<const floatx4*>(src + sl * sstride + 4);
+      for (int sl = 1; sl < nslices; sl += 8) {  // eight slices in flight
+        floatx4 u0[8], u1[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const float* p = src + min(sl + u, nslices - 1) * sstride;
+          u0[u] = *reinterpret_cast<const floatx4*>(p);
+          u1[u] = *reinterpret_cast<const floatx4*>(p + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (sl + u < nslices) {
+            s0 += u0[u];
+            s1 += u1[u];
+          }
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -367,7 +439,7 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
     for (int e = 0; e < 8; ++e) o[e] = (bf16)v[e];
     *reinterpret_cast<bf16x8*>(tS + toff<64, tpitch<64>()>(pr, pk)) = o;
   };
-  for (int st = 0; st < nsteps; ++st) {
+  for (int st = st0; st < st1; ++st) {
     lds_barrier();  // the previous step's reads of both buffers are done (st = 0: the ring's, and s_dcb)
     if (st <= kb) {
       store_piece(tS0, kb, st, pS0);
@@ -377,7 +449,7 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
       store_piece(tS1, kb + st, kb, pS1);
       tstage_store<64, NP, 512, PI>(sC, tBC1);
     }
-    if (st + 1 < nsteps) fetch(st + 1);
+    if (st + 1 < st1) fetch(st + 1);
     lds_barrier();
     lane = opaque_lane();
     hh = lane >> 5;
@@ -400,23 +472,7 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
       }
     }
   }
-  if (tok) {
-    const int64_t row = (int64_t)(ci.row0 + t) * brow + (int64_t)g * d.N;
-#pragma unroll
-    for (int q = 0; q < NTW; ++q) {
-      const int nt = nh * NTW + q;
-      if (nt >= NT) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n0 = 32 * nt + 8 * r + 4 * hh;
-        if (n0 >= d.N) continue;
-        bf16x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (bf16)acc[q][4 * r + e];
-        *reinterpret_cast<bf16x4*>((brole ? dB : dC) + row + n0) = o;
-      }
-    }
-  }
+  put();
 }
 
 // ---------------------------------------------------------------------------
@@ -437,13 +493,16 @@ template <int PT, int NT>
 static hipError_t bwd_gemm_t(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dB, void* dC,
                              hipStream_t s) {
   ensure_lds(k_bwd_gemm<PT, NT>, GemmCfg<PT, NT>::bytes);
-  const int nbq = d.Qpad / 64;
-  hipLaunchKernelGGL((k_bwd_gemm<PT, NT>), dim3((d.max_chunks + 7) / 8 * 8 * nbq, d.G), dim3(512), (GemmCfg<PT, NT>::bytes), s,
+  const int nbq = d.Qpad / 64, nz = (d.hpg + b.gemm_hslice - 1) / b.gemm_hslice;
+  const bool sliced = nz > 1 && !d.da_only;  // (a decay-only pass has no tile terms and nothing to sum)
+  hipLaunchKernelGGL((k_bwd_gemm<PT, NT>), dim3((d.max_chunks + 7) / 8 * 8 * nbq, d.G, sliced ? b.gemm_parts : nz), dim3(512),
+                     (GemmCfg<PT, NT>::bytes), s,
                      d, b.chunks, b.cs, in.dt, reinterpret_cast<const bf16*>(in.x),
                      reinterpret_cast<const bf16*>(dy), reinterpret_cast<const bf16*>(b.hin), b.hin_lo, b.dst16,
                      reinterpret_cast<const bf16*>(in.B), reinterpret_cast<const bf16*>(in.C), b.dS_tiles,
                      b.dS_tiles16, b.nslices, b.dS_fix, b.fast, b.dcs_off, reinterpret_cast<bf16*>(dB),
-                     reinterpret_cast<bf16*>(dC), b.tz_gam, b.xdy);
+                     reinterpret_cast<bf16*>(dC), b.tz_gam, b.xdy, b.gemm_hslice, b.gemm_tsteps, sliced ? b.dB_part : nullptr,
+                     sliced ? b.dC_part : nullptr);
   return hipGetLastError();
 }
 

@@ -32,8 +32,29 @@ struct Plan {
   int f32_fbatch, f32_bbatch, f32_rhs, f32_rsl;  // fp32: units per batch (forward, backward), row slices
   int fused_bwd, nrowg;
   int rows_chunk;  // fused path: the chunk-resident row kernel (k_bwd_rows) instead of k_bwd_gemm
+  int gemm_hslice, gemm_tsteps, gemm_parts;  // fused path: SsdBufs
   int head_bwd;    // fused path, one head per group: k_bwd_head in place of the column and row kernels
 };
+
+// k_bwd_gemm's slices. Its blocks (one per CU) walk a group's heads one after the other and then the chunk's tile
+// terms; where they fill a quarter of the chip or less, slices of the heads and the tile terms run side by side and
+// one more launch sums their partials. Forward and backward at P = 64, N = 128, whole / sliced, us:
+//   up to 32 blocks, four slices (more cost more to sum than they save) and one per tile step: 24 heads, chunk 256:
+//     256 tokens 117 / 81, 2048 tokens 146 / 120; 64 heads, 64 tokens 136 / 72; 8 heads, 512 tokens 78 / 69; below 6
+//     heads nothing (49 / 49 at 4)
+//   up to 64, two slices or three and one for the tile terms: 24 heads 160 / 141 (8 x 512 tokens 140 / 122), 64 heads
+//     277 / 229; 8 heads 97 / 99, so from 16 heads
+//   more: 96 blocks of 16 heads 140 / 142, 120 of 12 heads 119 / 126, 128 of 64 heads 425 / 407: whole
+void gemm_slices(const SsdDims& d, int* hslice, int* tsteps, int* parts) {
+  const int nb = d.Qpad / SSD_BLK;
+  const int64_t blocks = (int64_t)d.max_chunks * d.G * nb;
+  const bool few = blocks <= 32 && d.hpg >= 6;
+  int nz = few ? std::min(4, d.hpg / 2) : blocks <= 64 && d.hpg >= 16 ? (d.hpg >= 36 ? 3 : 2) : 1;
+  *hslice = (d.hpg + nz - 1) / nz;
+  nz = (d.hpg + *hslice - 1) / *hslice;
+  *tsteps = few ? 1 : nb;
+  *parts = nz > 1 ? nz + (nb + *tsteps - 1) / *tsteps : 1;
+}
 
 // `tight`: the plan with the smallest forward workspaces (wide bf16 heads whole, fp32 S tiles in the chunk
 // states' place).
@@ -131,6 +152,7 @@ int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
   if (ns > d.hpg) ns = d.hpg;
   p->hslice = (d.hpg + ns - 1) / ns;
   p->nslices = (d.hpg + p->hslice - 1) / p->hslice;
+  gemm_slices(d, &p->gemm_hslice, &p->gemm_tsteps, &p->gemm_parts);
   // the row kernel of the fused path; SSD_ROW_KERNEL=block or =chunk in the environment overrides the choice
   // (block: k_bwd_gemm everywhere; chunk: k_bwd_rows wherever its shape limits allow, any heads per group)
   const char* rk = getenv("SSD_ROW_KERNEL");
@@ -207,7 +229,8 @@ int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
   p->o_dD = take(MC * H * (d.Qpad / SSD_BLK) * sizeof(float));
   p->o_dA = take(MC * H * sizeof(float));
   const size_t bcn = (size_t)R * d.G * d.N * sizeof(float);
-  const int64_t nparts = f32 ? p->f32_rsl : p->nslices;
+  // (a fused plan's general kernels, for rows off the 16-byte grid, have nslices partials)
+  const int64_t nparts = f32 ? p->f32_rsl : std::max<int64_t>(p->nslices, p->fused_bwd ? p->gemm_parts : 1);
   p->o_dBp = nparts > 1 ? take(nparts * bcn) : 0;
   p->o_dCp = nparts > 1 ? take(nparts * bcn) : 0;
   p->o_bcb = f32 ? take(p->f32_bbatch * unit_bytes) : 0;
@@ -244,6 +267,9 @@ void bind_saved(const Plan& p, void* saved, SsdBufs* b) {
   b->norm_blocks = (int)p.norm_blocks;
   b->fused_bwd = p.fused_bwd;
   b->nrowg = p.nrowg;
+  b->gemm_hslice = p.gemm_hslice;
+  b->gemm_tsteps = p.gemm_tsteps;
+  b->gemm_parts = p.gemm_parts;
   b->ndcs = p.fused_bwd && !p.rows_chunk ? 2 : 1;
   b->rows_chunk = p.rows_chunk;
   b->dt_rep = p.o_dtrep ? reinterpret_cast<float*>(s + p.o_dtrep) : nullptr;
@@ -529,6 +555,17 @@ int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, 
     SSD_PHASE(tm, SSD_PH_NORM_BWD, launch_gated_norm_bwd(p.dtype, d, b, in, a->dy, a->dz, s));
     dY = b.dyp;
   }
+  // dB / dC of the head slices
+  const int nparts = p.dtype == SSD_DTYPE_F32    ? p.f32_rsl
+                     : !fused                    ? (int)p.nslices
+                     : (head || b.rows_chunk)    ? 1
+                                                 : p.gemm_parts;
+  auto reduce_bc = [&](const PhaseTimer& t) -> int {
+    if (nparts > 1)
+      SSD_PHASE(t, SSD_PH_BWD_REDUCE_BC,
+                launch_reduce_slices(p.dtype, d.R * d.G * d.N, nparts, b.dB_part, b.dC_part, a->dB, a->dC, s));
+    return SSD_OK;
+  };
   // One backward of the scan for (dd, bb, ii): the state pass (unless skipped: dst is then the one a
   // previous pass left in the scratch), the column / row phases and the finish.
   auto scan_bwd = [&](const SsdDims& dd, const SsdBufs& bb, const SsdIn& ii, const PhaseTimer& t, bool state_pass,
@@ -577,15 +614,7 @@ int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, 
       SSD_PHASE(t, SSD_PH_BWD_ROW, launch_bwd_row(dd, bb, ii, dY, a->dC, s));
     }
     SSD_PHASE(t, SSD_PH_BWD_FINISH, launch_bwd_finish(p.dtype, dd, bb, ii, ddt, dA_tok, da32, s));
-    const int nparts = p.dtype == SSD_DTYPE_F32 ? p.f32_rsl : (fused ? 1 : (int)p.nslices);
-    if (nparts > 1) {
-      const int64_t nelem = dd.R * dd.G * dd.N;
-      SSD_TRY(t.begin(SSD_PH_BWD_REDUCE_BC));
-      SSD_TRY(launch_reduce_slices(p.dtype, nelem, nparts, bb.dB_part, a->dB, s));
-      SSD_TRY(launch_reduce_slices(p.dtype, nelem, nparts, bb.dC_part, a->dC, s));
-      SSD_TRY(t.end(SSD_PH_BWD_REDUCE_BC));
-    }
-    return SSD_OK;
+    return reduce_bc(t);
   };
   // The reference's dA in the drop setting: the gamma path's alone, the decay gradient of
   // SSD(gamma x, a, B, C) over its own states (h_in of the gamma path, hgam).
@@ -637,7 +666,7 @@ int ssd_bwd(const ssd_desc_t* desc, const ssd_bwd_args_t* a, const void* saved, 
       SSD_PHASE(tm, SSD_PH_TRAPZ_GAMMA, launch_bwd_gemm(dg, bg, ig, dY, a->dB, a->dC, s));
     }
     SSD_PHASE(tm, SSD_PH_BWD_FINISH, launch_bwd_finish(p.dtype, dm, b, in, b.tz_ddt, nullptr, b.tz_da, s));
-    st = SSD_OK;
+    st = reduce_bc(tm);
   } else {
     if (d.trapz == SSD_TRAPZ_DROP_BETA_DA) {
       // (the column / row path) a backward of the gamma path that computes the decay gradient only (the

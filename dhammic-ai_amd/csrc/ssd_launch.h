@@ -152,8 +152,8 @@ hipError_t launch_trapz_grads(int dtype, const SsdDims& d, const SsdBufs& b, con
                               void* dA, hipStream_t s);
 
 // ssd_reduce.hip
-hipError_t launch_reduce_slices(int dtype, int64_t nelem, int nslices, const float* part, void* out,
-                                hipStream_t s);
+hipError_t launch_reduce_slices(int dtype, int64_t nelem, int nslices, const float* part0, const float* part1,
+                                void* out0, void* out1, hipStream_t s);
 // dA / dD per head and the norm weight's gradient (out = sum of part's nblocks rows of width) in one launch;
 // either side may be absent (dA_head = dD = nullptr, or out = nullptr)
 hipError_t launch_reduce_tail(const SsdDims& d, const SsdBufs& b, float* dA_head, float* dD, int nblocks, int width,

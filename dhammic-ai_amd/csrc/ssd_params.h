@@ -67,8 +67,8 @@ struct SsdBufs {
   float* xdx;              // [max_chunks][H][Qpad]
   float* dD_part;          // [max_chunks][H][Qpad/64]
   float* dA_part;          // [max_chunks][H]
-  float* dB_part;          // [nslices][R][G][N] (column / row kernels)
-  float* dC_part;          // [nslices][R][G][N]
+  float* dB_part;          // [head slices][R][G][N] (bf16 column / row kernels, fp32 rows, k_bwd_gemm)
+  float* dC_part;          // the same
   float* dS_tiles;         // fused path: [nslices][max_chunks][G][nb*nb][64][64] head-summed dS
   bf16* dS_tiles16;        // the same in bf16 when one head slice covers each group (nslices == 1; the row
                            // kernel rounds the tiles to bf16 for its products anyway); dS_tiles then nullptr
@@ -102,6 +102,7 @@ struct SsdBufs {
   int npass_blk, nslices, hslice, norm_blocks;
   int fused_bwd;           // 1: k_bwd_main + k_bwd_gemm (bf16), 0: column / row kernels
   int ndcs;                // dcs_off partials
+  int gemm_hslice, gemm_tsteps, gemm_parts;  // k_bwd_gemm: heads and tile steps per block, partial sums (1: none)
   int rows_chunk;          // fused path: k_bwd_rows builds dB / dC (else k_bwd_gemm)
   int nrowg;               // rowG partials (column sets of the fused path, else 1)
 };

@@ -3,27 +3,32 @@
 #include "ssd_launch.h"
 
 // out[i] = sum_s part[s][i], s = 0..nslices-1 in order.
+// Two sums of one shape per launch (dB and dC).
 template <typename T>
-__global__ void k_reduce_slices(int64_t nelem, int nslices, const float* __restrict__ part, T* __restrict__ out) {
+__global__ void k_reduce_slices(int64_t nelem, int nslices, const float* __restrict__ part0,
+                                const float* __restrict__ part1, T* __restrict__ out0, T* __restrict__ out1) {
+  const float* part = blockIdx.y ? part1 : part0;
+  T* out = blockIdx.y ? out1 : out0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nelem; i += (int64_t)gridDim.x * blockDim.x) {
     float acc = 0.0f;
+#pragma unroll 8
     for (int s = 0; s < nslices; ++s) acc += part[(int64_t)s * nelem + i];
     out[i] = from_f<T>(acc);
   }
 }
 
-hipError_t launch_reduce_slices(int dtype, int64_t nelem, int nslices, const float* part, void* out,
-                                hipStream_t s) {
+hipError_t launch_reduce_slices(int dtype, int64_t nelem, int nslices, const float* part0, const float* part1,
+                                void* out0, void* out1, hipStream_t s) {
   int64_t blocks64 = (nelem + 255) / 256;
   if (blocks64 > 65536) blocks64 = 65536;
   if (blocks64 < 1) blocks64 = 1;
   const unsigned blocks = (unsigned)blocks64;
   if (dtype == 1)
-    hipLaunchKernelGGL(k_reduce_slices<bf16>, dim3(blocks), dim3(256), 0, s, nelem, nslices, part,
-                       reinterpret_cast<bf16*>(out));
+    hipLaunchKernelGGL(k_reduce_slices<bf16>, dim3(blocks, 2), dim3(256), 0, s, nelem, nslices, part0, part1,
+                       reinterpret_cast<bf16*>(out0), reinterpret_cast<bf16*>(out1));
   else
-    hipLaunchKernelGGL(k_reduce_slices<float>, dim3(blocks), dim3(256), 0, s, nelem, nslices, part,
-                       reinterpret_cast<float*>(out));
+    hipLaunchKernelGGL(k_reduce_slices<float>, dim3(blocks, 2), dim3(256), 0, s, nelem, nslices, part0, part1,
+                       reinterpret_cast<float*>(out0), reinterpret_cast<float*>(out1));
   return hipGetLastError();
 }
 
