@@ -387,7 +387,10 @@ int fwd_impl(Plan& p, const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* sav
             launch_chunk_cumsum(p.dtype, d, b, a->A, a->dt, a->D, desc->want_A_cumsum ? a->A_cumsum_out : nullptr, s));
   // the factorised forward scan (bf16, 16-byte rows) computes S = C B^T per chunk and group anyway: in the
   // trapezoidal mode it also writes the per-token cb = C_t . B_t (S's diagonal) and D per token
-  const bool fwd_fact = scan_fwd_chunk_supported(p.dtype, d) && d.vec_x && d.vec_bc;
+  // Halves of wide heads take the exact kernel with S in fp32 (ssd_scan_fwd_chunk.hip): the factorised one would
+  // round S and x once more than the general kernel does for the whole head.
+  const bool fwd_fused = scan_fwd_chunk_supported(p.dtype, d) && d.vec_x && d.vec_bc;
+  const bool fwd_pairs = fwd_fused && d.hs, fwd_fact = fwd_fused && !d.hs;
   b.tz_cb_fwd = d.trapz && fwd_fact ? 1 : 0;
   if (d.trapz) {
     SSD_TRY(tm.begin(SSD_PH_TRAPZ_PREP));
@@ -425,7 +428,9 @@ int fwd_impl(Plan& p, const ssd_desc_t* desc, const ssd_fwd_args_t* a, void* sav
     if (b.tz_cb_fwd) SSD_TRY(launch_trapz_dtok(d, b, Dk, s));
     SSD_TRY(launch_scan_fwd_chunk(d, b, in, yout, b.fast, s));
     SSD_TRY(tm.end(SSD_PH_FWD_SCAN));
-  } else if (p.dtype == SSD_DTYPE_F32)
+  } else if (fwd_pairs)
+    SSD_PHASE(tm, SSD_PH_FWD_SCAN, launch_scan_fwd_pairs(d, b, in, yout, s));
+  else if (p.dtype == SSD_DTYPE_F32)
     SSD_PHASE(tm, SSD_PH_FWD_SCAN, launch_f32_scan(d, b, in, yout, s));
   else
     SSD_PHASE(tm, SSD_PH_FWD_SCAN, launch_chunk_scan_fwd(d, b, in, yout, s));

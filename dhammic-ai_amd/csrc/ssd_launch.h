@@ -61,6 +61,7 @@ size_t lds_scan_fwd_chunk(const SsdDims& d);
 // of the factorised kernel
 hipError_t launch_scan_fwd_chunk(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, const int32_t* fast,
                                  hipStream_t s);
+hipError_t launch_scan_fwd_pairs(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s);
 
 // ssd_scan_fwd_fact.hip (same shapes): the factorised-decay forward scan, exact for the (chunk, head)
 // pairs k_chunk_cumsum flags 1; the others are rewritten by launch_scan_fwd_chunk(..., b.fast, ...)

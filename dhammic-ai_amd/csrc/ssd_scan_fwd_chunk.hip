@@ -22,6 +22,11 @@
 // This exact per-element form runs as the fixup of the factorised kernel
 // (ssd_scan_fwd_fact.hip): with `fast` given, only blocks whose head slice
 // holds a (chunk, head) flagged 0 run, and they rewrite their whole slice.
+// S32 (halves of wide heads, whole grid): S^T stays in fp32 registers, so M is the only operand that is
+// rounded, as in the general kernel that takes such heads whole. The factorised kernel rounds S' and the
+// scaled x: y of the reference op with 128-column heads is 2.87e-3 from 64 bits there, 2.37e-3 here.
+// Price, forward and backward at B=4 L=2048 H=16 P=128 N=64 chunk 256 with the norm: 254 -> 288 us (whole heads on
+// the general kernels: 605).
 #include <algorithm>
 
 #include "ssd_launch.h"
@@ -57,7 +62,7 @@ struct FwdStage {
 #define SSD_FWD_CHUNK_ARGS d, hslice, nslices, chunks, cs, hin, x, dt, Bm, Cm, Dv, y, fast, Dtok
 
 // The work of block `bid`: (chunk bid % max_chunks, group and head slice bid / max_chunks).
-template <int PT, int NT, int NB>
+template <int PT, int NT, int NB, bool S32>
 __device__ __forceinline__ void scan_fwd_chunk_block(int bid, SSD_FWD_CHUNK_PARAMS) {
   constexpr int PP = 32 * PT, NP = 32 * NT;
   constexpr int XT = tsize<64, PP>(), CT = tsize<64, NP>();
@@ -112,7 +117,8 @@ __device__ __forceinline__ void scan_fwd_chunk_block(int bid, SSD_FWD_CHUNK_PARA
   __syncthreads();
 
   // ---- S^T units: rows s (block j half sh), lanes l (quadrant) ----
-  bf16x8 S[kUnits][2];
+  bf16x8 S[S32 ? 1 : kUnits][2];
+  floatx16 Sf[S32 ? kUnits : 1];
 #pragma unroll
   for (int u = 0; u < kUnits; ++u) {
     floatx16 sacc;
@@ -134,8 +140,12 @@ __device__ __forceinline__ void scan_fwd_chunk_block(int bid, SSD_FWD_CHUNK_PARA
         mfma(sacc, bv, tld8<NP>(Ct + qi[q] * CT, 32 * qlh[q] + (lane & 31), n0));
       }
     }
-    S[u][0] = acc_frag(sacc, 0);
-    S[u][1] = acc_frag(sacc, 1);
+    if constexpr (S32) {
+      Sf[u] = sacc;
+    } else {
+      S[u][0] = acc_frag(sacc, 0);
+      S[u][1] = acc_frag(sacc, 1);
+    }
   }
 
   // ---- per-head loop with the next head's inputs in flight ----
@@ -159,10 +169,12 @@ __device__ __forceinline__ void scan_fwd_chunk_block(int bid, SSD_FWD_CHUNK_PARA
   load_head(h_lo);
   for (int h = h_lo; h < h_hi; ++h) {
     lane = opaque_lane();
+    if constexpr (!S32) {
 #pragma unroll
-    for (int u = 0; u < kUnits; ++u) {
-      launder(S[u][0]);
-      launder(S[u][1]);
+      for (int u = 0; u < kUnits; ++u) {
+        launder(S[u][0]);
+        launder(S[u][1]);
+      }
     }
     __syncthreads();  // the previous head's LDS reads are done
 #pragma unroll
@@ -213,7 +225,12 @@ __device__ __forceinline__ void scan_fwd_chunk_block(int bid, SSD_FWD_CHUNK_PARA
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const float dd = cs_l - css[v];
-          float mv = (float)S[u][v >> 3][v & 7] * exp2_fast(clamp_med3(dd, -SSD_T2, SSD_T2)) * dts[v];
+          float sv;
+          if constexpr (S32)
+            sv = Sf[u][v];
+          else
+            sv = (float)S[u][v >> 3][v & 7];
+          float mv = sv * exp2_fast(clamp_med3(dd, -SSD_T2, SSD_T2)) * dts[v];
           if (diag && acc_row(v, lane) + (d.trapz ? 1 : 0) > (lane & 31)) mv = 0.0f;  // trapz: strict
           m[v] = mv;
         }
@@ -251,11 +268,11 @@ __device__ __forceinline__ void scan_fwd_chunk_block(int bid, SSD_FWD_CHUNK_PARA
 // block taking the units blockIdx.x + k gridDim.x, reading all their flags at once and running only the
 // units holding a flagged head (a block per unit that mostly exits at once costs a launch wave per
 // 256 of them).
-template <int PT, int NT, int NB>
+template <int PT, int NT, int NB, bool S32>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 k_scan_fwd_chunk(int total, SSD_FWD_CHUNK_PARAMS) {
-  if (!fast) {
-    scan_fwd_chunk_block<PT, NT, NB>(blockIdx.x, SSD_FWD_CHUNK_ARGS);
+  if (S32 || !fast) {
+    scan_fwd_chunk_block<PT, NT, NB, S32>(blockIdx.x, SSD_FWD_CHUNK_ARGS);
     return;
   }
   __shared__ int s_need[SSD_FIX_UNITS];
@@ -273,7 +290,7 @@ k_scan_fwd_chunk(int total, SSD_FWD_CHUNK_PARAMS) {
   for (int k = 0; k < per; ++k) {
     if (!s_need[k]) continue;
     __syncthreads();  // the previous unit's LDS reads are done
-    scan_fwd_chunk_block<PT, NT, NB>(blockIdx.x + k * gridDim.x, SSD_FWD_CHUNK_ARGS);
+    scan_fwd_chunk_block<PT, NT, NB, S32>(blockIdx.x + k * gridDim.x, SSD_FWD_CHUNK_ARGS);
   }
 }
 
@@ -295,7 +312,7 @@ size_t lds_scan_fwd_chunk(const SsdDims& d) {
   }
 }
 
-template <int PT, int NT, int NB>
+template <int PT, int NT, int NB, bool S32>
 static hipError_t scan_fwd_chunk_t(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y,
                                    const int32_t* fast, hipStream_t s) {
   // heads per block: about four blocks per CU over the grid
@@ -303,27 +320,28 @@ static hipError_t scan_fwd_chunk_t(const SsdDims& d, const SsdBufs& b, const Ssd
   int ns = (1024 + per - 1) / per;
   if (ns < 1) ns = 1;
   if (ns > d.hpg) ns = d.hpg;
-  const int hslice = (d.hpg + ns - 1) / ns;
+  int hslice = (d.hpg + ns - 1) / ns;
+  if (S32 && hslice < 2) hslice = 2;  // the halves of a head share S
   ns = (d.hpg + hslice - 1) / hslice;
   const size_t lds = FwdLds<PT, NT>::bytes(NB);
-  ensure_lds(k_scan_fwd_chunk<PT, NT, NB>, lds);
+  ensure_lds(k_scan_fwd_chunk<PT, NT, NB, S32>, lds);
   const int blocks = d.max_chunks * d.G * ns;
   const int grid = fast ? std::max(std::min(blocks, 256), (blocks + SSD_FIX_UNITS - 1) / SSD_FIX_UNITS) : blocks;
-  hipLaunchKernelGGL((k_scan_fwd_chunk<PT, NT, NB>), dim3(grid), dim3(256), lds, s, blocks, d, hslice, ns,
+  hipLaunchKernelGGL((k_scan_fwd_chunk<PT, NT, NB, S32>), dim3(grid), dim3(256), lds, s, blocks, d, hslice, ns,
                      b.chunks, b.cs, reinterpret_cast<const bf16*>(b.hin), reinterpret_cast<const bf16*>(in.x), in.dt,
                      reinterpret_cast<const bf16*>(in.B), reinterpret_cast<const bf16*>(in.C), in.D,
                      reinterpret_cast<bf16*>(y), fast, b.Dtok);
   return hipGetLastError();
 }
 
-template <int PT, int NT>
+template <int PT, int NT, bool S32 = false>
 static hipError_t scan_fwd_chunk_nb(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y,
                                     const int32_t* fast, hipStream_t s) {
   switch (d.Qpad / 64) {
-    case 1: return scan_fwd_chunk_t<PT, NT, 1>(d, b, in, y, fast, s);
-    case 2: return scan_fwd_chunk_t<PT, NT, 2>(d, b, in, y, fast, s);
-    case 3: return scan_fwd_chunk_t<PT, NT, 3>(d, b, in, y, fast, s);
-    default: return scan_fwd_chunk_t<PT, NT, 4>(d, b, in, y, fast, s);
+    case 1: return scan_fwd_chunk_t<PT, NT, 1, S32>(d, b, in, y, fast, s);
+    case 2: return scan_fwd_chunk_t<PT, NT, 2, S32>(d, b, in, y, fast, s);
+    case 3: return scan_fwd_chunk_t<PT, NT, 3, S32>(d, b, in, y, fast, s);
+    default: return scan_fwd_chunk_t<PT, NT, 4, S32>(d, b, in, y, fast, s);
   }
 }
 
@@ -336,5 +354,14 @@ hipError_t launch_scan_fwd_chunk(const SsdDims& d, const SsdBufs& b, const SsdIn
     case 21: return scan_fwd_chunk_nb<2, 1>(d, b, in, y, fast, s);
     case 22: return scan_fwd_chunk_nb<2, 2>(d, b, in, y, fast, s);
     default: return scan_fwd_chunk_nb<2, 4>(d, b, in, y, fast, s);
+  }
+}
+
+// Every (chunk, head) with S in fp32: the halves of 80- to 128-column heads, 40 to 64 columns each.
+hipError_t launch_scan_fwd_pairs(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s) {
+  switch (d.Npad / 32) {
+    case 1: return scan_fwd_chunk_nb<2, 1, true>(d, b, in, y, nullptr, s);
+    case 2: return scan_fwd_chunk_nb<2, 2, true>(d, b, in, y, nullptr, s);
+    default: return scan_fwd_chunk_nb<2, 4, true>(d, b, in, y, nullptr, s);
   }
 }
