@@ -18,6 +18,7 @@
 //   R: lane = s, registers over l                              (S of the backward, dS: M^T dy, dS^T C)
 // Tile (lt, st), st <= lt, of a unit (chunk, group) is number lt (lt + 1) / 2 + st.
 #include "ssd_launch.h"
+#include "ssd_stage.h"
 #include "ssd_tile.h"
 
 namespace {
@@ -48,22 +49,23 @@ __device__ __forceinline__ void st_tile(float* __restrict__ t, int lane, const f
 }
 
 // Rows [0, nrows) (valid below len) x [0, W) columns (valid below width) of a row-major tensor into LDS
-// (pitch floats per row), zeros elsewhere. Masked buffer loads, eight pieces per thread in flight.
+// (pitch floats per row), zeros elsewhere. Masked buffer loads, eight pieces per thread in flight; ssd_stage.h has
+// the addresses.
 template <int W, bool VEC>
 __device__ __forceinline__ void stage_rows_v(float* __restrict__ out, int pitch, const float* __restrict__ src,
                                              int64_t ld, int nrows, int len, int width) {
   constexpr int CPR = W / 4, NB = 8;
-  const int total = nrows * CPR;
-  for (int id0 = threadIdx.x; id0 < total; id0 += NB * blockDim.x) {
+  static_assert(64 % CPR == 0, "a wave holds whole rows");
+  const int total = nrows * CPR, nthr = blockDim.x;
+  for (int id0 = threadIdx.x; id0 < total; id0 += NB * nthr) {
     floatx4 v[NB];
-    // (the resource's base moves with the rows: offsets stay below 2 GiB)
-    const int r0 = __builtin_amdgcn_readfirstlane(id0 / CPR);
-    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(src + (int64_t)r0 * ld);
+    const int w0 = __builtin_amdgcn_readfirstlane(id0);
+    const int k = stage_col(id0, CPR), off = stage_off(id0, w0, CPR, ld);
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
-      const int id = id0 + q * blockDim.x, r = id / CPR, k = (id % CPR) * 4;
-      const bool ok = id < total && r < len;
-      const int off = (r - r0) * (int)ld + k;
+      const int id = id0 + q * nthr;
+      const bool ok = id < total && stage_row(id, CPR) < len;
+      const __amdgpu_buffer_rsrc_t rs = buf_rsrc(src + stage_base(w0, q, nthr, CPR) * ld);
       if constexpr (VEC) {
         v[q] = __builtin_bit_cast(
             floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, ok && k < width ? off * 4 : SSD_BUF_SIZE, 0, 0));
@@ -74,8 +76,8 @@ __device__ __forceinline__ void stage_rows_v(float* __restrict__ out, int pitch,
     }
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
-      const int id = id0 + q * blockDim.x, r = id / CPR, k = (id % CPR) * 4;
-      if (id < total) *reinterpret_cast<floatx4*>(out + r * pitch + k) = v[q];
+      const int id = id0 + q * nthr;
+      if (id < total) *reinterpret_cast<floatx4*>(out + stage_row(id, CPR) * pitch + k) = v[q];
     }
   }
 }

@@ -87,3 +87,22 @@ def test_noalloc_forward_with_tiles_in_parts():
     y1, f1, _ = na._noalloc(cfg, *args)
     assert torch.equal(y1, y0) and torch.equal(f1, f0)
     assert rel_err(y1, y0) <= TOL[torch.float32]
+
+
+def test_halves_of_wide_heads_at_the_largest_row_strides():
+    """36 600 heads of 128 columns: rows 18.7 MB apart, so that one 64-column half's rows span more than 2 GiB from
+    row 115 on. y of the last heads is that of the call on those heads alone."""
+    import kernels
+    H, L, k = 36600, 128, 8
+    g = torch.Generator(device=DEV).manual_seed(11)
+    x = torch.randn(1, L, H, 128, generator=g, device=DEV)
+    dt = torch.rand(1, L, H, generator=g, device=DEV) * 0.1
+    A = -torch.rand(H, generator=g, device=DEV) * 4 - 1
+    B, C = (torch.randn(1, L, 1, 16, generator=g, device=DEV) for _ in range(2))
+    with torch.no_grad():
+        y = kernels.ssd_scan_combined(x, dt, A, B, C, 256)
+        for lo in (0, H - k):
+            got = kernels.ssd_scan_combined(x[:, :, lo:lo + k].contiguous(), dt[:, :, lo:lo + k].contiguous(),
+                                            A[lo:lo + k].contiguous(), B, C, 256)
+            assert torch.equal(y[:, :, lo:lo + k], got)
+            assert y[:, 115:, lo:lo + k].abs().min() > 0
