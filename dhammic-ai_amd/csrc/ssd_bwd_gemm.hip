@@ -28,9 +28,11 @@
 // hit distinct banks.
 //
 // Few blocks (a short batch of one or two groups): the walk over the heads is a serial chain of ~2.2 us each and the
-// tile terms another one (each step sums the column slices' dS partials, eight in flight: 70 -> 58 us for 24 heads of
+// tile terms another one (each step sums the column slices' dS partials, several in flight: 70 -> 58 us for 24 heads of
 // one 256-token chunk), so both go to slices with fp32 partials of dB / dC (58 -> 22 us with the launch that sums
 // them; gemm_slices in ssd_capi.hip has the rule).
+#include <type_traits>
+
 #include "ssd_launch.h"
 #include "ssd_tile.h"
 
@@ -49,12 +51,17 @@ struct GemmCfg {
   static constexpr int kRowDma = XT / 512;
   static constexpr int kPerWave = (2 * kTileDma + 2 * kRowDma) / 4 + 1;
   static_assert((2 * kTileDma + 2 * kRowDma) % 4 == 0, "DMA split");
+  // Waves per SIMD to leave registers for: two blocks per CU (at most 128 VGPRs) where two rings fit its 160 KB of LDS
+  // and the registers suffice (the 128-column dC / dB accumulators of NT = 4 take 158 and more).
+  static constexpr int kWaves = NT <= 2 && 2 * (bytes + 256) <= 160 * 1024 ? 4 : 2;
 };
 
 }  // namespace
 
-template <int PT, int NT>
-__global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __restrict__ chunks,
+// MULTI: fp32 dS partials of several column slices (nslices > 1), summed here, and this kernel's own slices. Whole
+// bf16 dS tiles (one column slice) take the other variant, which holds none of the registers the partials need.
+template <int PT, int NT, bool MULTI>
+__global__ void __launch_bounds__(512, (GemmCfg<PT, NT>::kWaves)) k_bwd_gemm(SsdDims d, const ChunkInfo* __restrict__ chunks,
                                                   const float* __restrict__ cs, const float* __restrict__ dt,
                                                   const bf16* __restrict__ x, const bf16* __restrict__ dy,
                                                   const bf16* __restrict__ hin, const uint8_t* __restrict__ hin_lo,
@@ -94,7 +101,7 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
   const int MC = d.max_chunks, Qpad = d.Qpad;
   // this block's heads: all of the group's, then the tile terms; or (dB_part set) slice z of hslice heads, with more
   // slices for tsteps steps of the tile terms each
-  const bool sliced = dB_part != nullptr;
+  const bool sliced = MULTI && dB_part != nullptr;
   const int hz = blockIdx.z * hslice, nhd = max(0, min(hslice, d.hpg - hz));
   const int h0 = g * d.hpg + hz;
 
@@ -183,12 +190,12 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
   const int64_t tile0 = ((int64_t)c * d.G + g) * nb * nb * 4096;
   const int pid = threadIdx.x, pr = pid >> 3, pk = (pid & 7) * 8;  // this thread's piece of a tile
   const int nsteps = max(kb + 1, nbl - kb);
-  const __amdgpu_buffer_rsrc_t rS = buf_rsrc(dS16 ? (const void*)(dS16 + tile0) : (const void*)dS);
+  const __amdgpu_buffer_rsrc_t rS = buf_rsrc(MULTI ? (const void*)dS : (const void*)(dS16 + tile0));
   bf16x8 pS0, pS1;
   TileStage<64, NP, 512> sB, sC;
   auto fetch = [&](int st) {
     const bool ok0 = st <= kb, ok1 = kb + st < nbl;
-    if (dS16) {
+    if (!MULTI) {
       pS0 = buf_ld16(rS, (int)((((int64_t)kb * nb + st) * 4096 + pr * 64 + pk) * 2), ok0);
       pS1 = buf_ld16(rS, (int)((((int64_t)(kb + st) * nb + kb) * 4096 + pr * 64 + pk) * 2), ok1);
     }
@@ -394,28 +401,40 @@ __global__ void __launch_bounds__(512) k_bwd_gemm(SsdDims d, const ChunkInfo* __
   // heads' dS and (trapezoidal mode, tile (kb, kb)) the diagonal sum_h gamma (x_t . dy_t)
   auto store_piece = [&](bf16* tS, int ti, int tj, const bf16x8& pre) {
     float v[8];
-    if (dS16) {
+    if constexpr (!MULTI) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = (float)pre[e];
     } else {
-      const float* src = dS + tile0 + ((int64_t)ti * nb + tj) * 4096 + pr * 64 + pk;
-      floatx4 s0 = *reinterpret_cast<const floatx4*>(src);
-      floatx4 s1 = *reinterpret_cast<const floatx4*>(src + 4);
-      for (int sl = 1; sl < nslices; sl += 8) {  // eight slices in flight
-        floatx4 u0[8], u1[8];
+      // (uniform bases, one per slice: the lane's offset is the same in all of them)
+      const float* src = dS + tile0 + ((int64_t)ti * nb + tj) * 4096;
+      const int po = (pr * 64 + pk) * 4;
+      auto ld = [&](int slc, floatx4& a0, floatx4& a1) {
+        const __amdgpu_buffer_rsrc_t r = buf_rsrc(src + slc * sstride);
+        a0 = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, po, 0, 0));
+        a1 = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, po + 16, 0, 0));
+      };
+      floatx4 s0, s1;
+      ld(0, s0, s1);
+      // the other slices in order, up to six of them in flight (eight take 135 VGPRs: one block per CU)
+      int sl = 1;
+      auto add = [&](auto n) {
+        constexpr int U = decltype(n)::value;
+#pragma unroll 1
+        for (; sl + U <= nslices; sl += U) {
+          floatx4 u0[U], u1[U];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const float* p = src + min(sl + u, nslices - 1) * sstride;
-          u0[u] = *reinterpret_cast<const floatx4*>(p);
-          u1[u] = *reinterpret_cast<const floatx4*>(p + 4);
-        }
+          for (int u = 0; u < U; ++u) ld(sl + u, u0[u], u1[u]);
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (sl + u < nslices) {
+          for (int u = 0; u < U; ++u) {
             s0 += u0[u];
             s1 += u1[u];
           }
-      }
+        }
+      };
+      add(std::integral_constant<int, 6>{});
+      add(std::integral_constant<int, 3>{});
+      add(std::integral_constant<int, 2>{});
+      add(std::integral_constant<int, 1>{});
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         v[e] = s0[e];
@@ -489,14 +508,14 @@ size_t lds_bwd_gemm(const SsdDims& d) {
   }
 }
 
-template <int PT, int NT>
-static hipError_t bwd_gemm_t(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dB, void* dC,
+template <int PT, int NT, bool MULTI>
+static hipError_t bwd_gemm_m(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dB, void* dC,
                              hipStream_t s) {
-  ensure_lds(k_bwd_gemm<PT, NT>, GemmCfg<PT, NT>::bytes);
+  ensure_lds(k_bwd_gemm<PT, NT, MULTI>, GemmCfg<PT, NT>::bytes);
   const int nbq = d.Qpad / 64, nz = (d.hpg + b.gemm_hslice - 1) / b.gemm_hslice;
-  const bool sliced = nz > 1 && !d.da_only;  // (a decay-only pass has no tile terms and nothing to sum)
-  hipLaunchKernelGGL((k_bwd_gemm<PT, NT>), dim3((d.max_chunks + 7) / 8 * 8 * nbq, d.G, sliced ? b.gemm_parts : nz), dim3(512),
-                     (GemmCfg<PT, NT>::bytes), s,
+  const bool sliced = MULTI && nz > 1 && !d.da_only;  // (a decay-only pass has no tile terms and nothing to sum)
+  hipLaunchKernelGGL((k_bwd_gemm<PT, NT, MULTI>), dim3((d.max_chunks + 7) / 8 * 8 * nbq, d.G, sliced ? b.gemm_parts : nz),
+                     dim3(512), (GemmCfg<PT, NT>::bytes), s,
                      d, b.chunks, b.cs, in.dt, reinterpret_cast<const bf16*>(in.x),
                      reinterpret_cast<const bf16*>(dy), reinterpret_cast<const bf16*>(b.hin), b.hin_lo, b.dst16,
                      reinterpret_cast<const bf16*>(in.B), reinterpret_cast<const bf16*>(in.C), b.dS_tiles,
@@ -504,6 +523,14 @@ static hipError_t bwd_gemm_t(const SsdDims& d, const SsdBufs& b, const SsdIn& in
                      reinterpret_cast<bf16*>(dC), b.tz_gam, b.xdy, b.gemm_hslice, b.gemm_tsteps, sliced ? b.dB_part : nullptr,
                      sliced ? b.dC_part : nullptr);
   return hipGetLastError();
+}
+
+// (the row kernel's slices come with several column slices: gemm_slices splits at 64 blocks or fewer and 6 heads or
+// more, where the column side has four slices or one per head)
+template <int PT, int NT>
+static hipError_t bwd_gemm_t(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dB, void* dC,
+                             hipStream_t s) {
+  return b.dS_tiles ? bwd_gemm_m<PT, NT, true>(d, b, in, dy, dB, dC, s) : bwd_gemm_m<PT, NT, false>(d, b, in, dy, dB, dC, s);
 }
 
 hipError_t launch_bwd_gemm(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dB, void* dC,
