@@ -80,9 +80,10 @@ __global__ void __launch_bounds__(512, (GemmCfg<PT, NT>::kWaves)) k_bwd_gemm(Ssd
   extern __shared__ __align__(16) unsigned char smem[];
   // block -> (chunk, 64-token block kb): the nb blocks of a chunk are consecutive in
   // dispatch order and share an XCD (same index mod 8), so each head's h_in / dst
-  // tiles come from HBM once and from that XCD's L2 for the other blocks
+  // tiles come from HBM once and from that XCD's L2 for the other blocks. The chunks of
+  // the next group or slice go on where the last one's ended, mod 8: all XCDs get as many, also of few chunks.
   const int nbq = d.Qpad / 64;
-  const int x8 = blockIdx.x & 7, rr = blockIdx.x >> 3;
+  const int x8 = (blockIdx.x - d.max_chunks * (blockIdx.y + d.G * blockIdx.z)) & 7, rr = blockIdx.x >> 3;
   const int kb = rr % nbq;
   const int c = (rr / nbq) * 8 + x8, g = blockIdx.y;
   if (c >= d.max_chunks) return;

@@ -45,6 +45,9 @@ struct Plan {
 //   up to 64, two slices or three and one for the tile terms: 24 heads 160 / 141 (8 x 512 tokens 140 / 122), 64 heads
 //     277 / 229; 8 heads 97 / 99, so from 16 heads
 //   more: 96 blocks of 16 heads 140 / 142, 120 of 12 heads 119 / 126, 128 of 64 heads 425 / 407: whole
+// With several groups (one chunk of 256 tokens, 64 heads in 2 / 4 / 8 groups 160 / 93, 119 / 90, 103 / 90; four
+// chunks in 4 groups 130 / 120) this holds because the kernel spreads groups and slices over the XCDs: on the chunks'
+// own XCDs the slices queued up (8 groups 153).
 void gemm_slices(const SsdDims& d, int* hslice, int* tsteps, int* parts) {
   const int nb = d.Qpad / SSD_BLK;
   const int64_t blocks = (int64_t)d.max_chunks * d.G * nb;

@@ -28,6 +28,9 @@ DEV, BF = "cuda", torch.bfloat16
     (1, 2048, 24, 64, 1, 32, 256, None),               # 32 blocks, the last of the first rule
     (1, 2304, 16, 64, 1, 32, 256, None),               # 36 blocks, two slices and one for the tile terms
     (2, 2048, 37, 32, 1, 64, 256, None),               # 64 blocks, 37 heads in slices of 13, 13 and 11
+    (1, 256, 48, 64, 8, 128, 256, None),               # one chunk of eight groups: blocks on every XCD
+    (1, 700, 18, 64, 3, 32, 256, None),                # three chunks of three groups, slices of 2
+    (9, 128, 16, 32, 2, 32, 128, None),                # nine chunks: a second round of XCDs, padded to 16
     (1, 900, 16, 64, 2, 64, 256, [0, 1, 1, 258, 900]),  # packed: a token, none, two chunks, a remainder
 ])
 def test_shapes(b, L, H, P, G, N, Q, cu):
