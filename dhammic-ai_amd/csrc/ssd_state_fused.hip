@@ -49,6 +49,7 @@ struct StateCfg {
   static constexpr int PERW = (UI + VI) / NPW;  // row DMAs per DMA wave and step
   static constexpr int D = PERW, D0 = PERW + 1; // DMAs per step: any DMA wave, DMA wave 0 (+ the factor row)
   static_assert(UI % NPW == 0 && VI % NPW == 0, "DMA split");
+  static_assert(NTHR <= 1024, "the largest block a launch takes");
   static constexpr int TP = 40;                 // s_tile row pitch (elements), 32 x 32 tiles
   // PT = 2: each wave owns all 64 p of 16 columns of the pair (four 16 x 16 MFMA tiles), so every
   // B / C element is scaled by one wave, not by both p-tile waves; other PT use 32 x 32 tiles
@@ -586,12 +587,16 @@ static void state_fused_nt(const SsdDims& d, const SsdBufs& b, const bf16* u, co
                            bf16* hst, uint8_t* hlo, const bf16* hin_in, const void* s_in, void* s_out, int state_bf16,
                            hipStream_t s, const Walk2& w2) {
   // at most half the CUs' worth of (head, sequence) walks: two blocks per unit, each over half the state
-  // columns (each reads the unit's x / dy rows; every walk is serial, so idle CUs are the larger loss)
-  const int nsplit = ((w2.fac ? 2 : 1) * d.H * d.nseq <= 128 && d.Npad / 32 >= 2) ? 2 : 1;
+  // columns (each reads the unit's x / dy rows; every walk is serial, so idle CUs are the larger loss). States of
+  // 128 x 128 always: one block's compute and DMA waves would be 20.
+  const bool few = (w2.fac ? 2 : 1) * d.H * d.nseq <= 128 && d.Npad / 32 >= 2;
+  const int nsplit = few || (PT == 4 && d.Npad == 128) ? 2 : 1;
   switch (d.Npad / 32 / nsplit) {
     case 1: state_fused_launch<PT, 1, FWD>(d, b, u, v, fac, hst, hlo, hin_in, s_in, s_out, state_bf16, s, nsplit, w2); break;
     case 2: state_fused_launch<PT, 2, FWD>(d, b, u, v, fac, hst, hlo, hin_in, s_in, s_out, state_bf16, s, nsplit, w2); break;
-    default: state_fused_launch<PT, 4, FWD>(d, b, u, v, fac, hst, hlo, hin_in, s_in, s_out, state_bf16, s, nsplit, w2);
+    default:
+      if constexpr (PT < 4)
+        state_fused_launch<PT, 4, FWD>(d, b, u, v, fac, hst, hlo, hin_in, s_in, s_out, state_bf16, s, nsplit, w2);
   }
 }
 

@@ -125,3 +125,45 @@ def test_forward_rounds_only_the_decayed_scores(P, N, chunk):
     err = ((y - ref).norm() / ref.norm()).item()
     print(P, N, chunk, err)
     assert err <= 2.6e-3, err
+
+
+@pytest.mark.parametrize("P,H,b,L,Q,cu", [
+    (104, 65, 2, 70, 64, None),                      # 130 (head, sequence) walks, two chunks
+    (88, 33, 1, 300, 128, [0, 1, 90, 90, 200, 300]),  # 165 walks of packed sequences, one of them empty
+    (120, 129, 1, 40, 256, None),
+])
+def test_whole_heads_with_128_state_columns(P, H, b, L, Q, cu):
+    """Heads that do not halve (P % 16 != 0), states of 128 x 128 padded, more walks than half the CUs: a block per
+    walk would need 1280 threads, so every walk is two blocks over half the columns."""
+    tp._check_ext(SsdShape(b, L, H, P, 1, 128, Q, cu_seqlens=cu), BF, with_z=False, seed=P, cu=cu, randw=True)
+
+
+def test_noalloc_whole_heads_with_128_state_columns():
+    """The first head count whose pairs do not fit the no-allocation scratch: whole heads with 128 x 128 states."""
+    import ctypes
+    import test_zz_no_alloc as na
+    from kernels import _capi as C_
+    from kernels import ssd_scan as ks
+    lib = C_.load()
+    cfg = ks._Cfg(chunk=64, a_mode=C_.SSD_A_PER_HEAD, nseq=1, varlen=False, state_code=C_.SSD_DTYPE_F32, want_acs=False,
+                  eps=1e-6)
+
+    def need(H):
+        d = ctypes.byref(ks._desc_of(cfg, (1, 64, H, 128), 1, 128, BF, True, True, False, False, False))
+        saved, fwd = (lib.ssd_workspace_bytes(d, k) for k in (C_.SSD_WS_SAVED, C_.SSD_WS_FWD_SCRATCH))
+        return (saved + 255) // 256 * 256 + fwd
+
+    H = next(h for h in range(129, 2000) if need(h) > C_.SSD_NOALLOC_SCRATCH_BYTES)
+    inp = {k: v.to(DEV) for k, v in make_inputs(SsdShape(1, 64, H, 128, 1, 128, 64), seed=1).items()}
+    args = (inp["x"].to(BF), inp["dt"], inp["A"], inp["B"].to(BF), inp["C"].to(BF), inp["D"], None, None, None, None)
+    y0, f0, _, _ = ks._forward(cfg, *args)
+    y1, f1, _ = na._noalloc(cfg, *args)
+    assert not torch.equal(y1, y0)  # (other kernels)
+    assert_close("y", y1, y0, TOL[BF])
+    assert_close("final", f1, f0, TOL[BF])
+
+
+@pytest.mark.parametrize("exact", tz.MODES, ids=tz.MODE_IDS)
+def test_trapezoidal_whole_heads_with_128_state_columns(exact):
+    tz.check(tz.make(1, 100, 70, 104, 1, 128, BF, seed=4), 64, exact, BF, oracle_device=DEV, oracle_dtype=torch.float32,
+             tag="whole P=104 N=128")
