@@ -26,7 +26,8 @@
 // rounded, as in the general kernel that takes such heads whole. The factorised kernel rounds S' and the
 // scaled x: y of the reference op with 128-column heads is 2.87e-3 from 64 bits there, 2.37e-3 here.
 // Price, forward and backward at B=4 L=2048 H=16 P=128 N=64 chunk 256 with the norm: 254 -> 288 us (whole heads on
-// the general kernels: 605).
+// the general kernels: 605). Up to 128-token chunks two blocks share a CU, where a lone one waits for its loads: 8 x 2048
+// tokens of 32 heads of 128 columns, 32 groups, N=16, chunk 64, the forward 355 -> 249 us (whole heads 285).
 #include <algorithm>
 
 #include "ssd_launch.h"
@@ -269,7 +270,7 @@ __device__ __forceinline__ void scan_fwd_chunk_block(int bid, SSD_FWD_CHUNK_PARA
 // units holding a flagged head (a block per unit that mostly exits at once costs a launch wave per
 // 256 of them).
 template <int PT, int NT, int NB, bool S32>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, S32 && NB <= 2 ? 2 : 1)))
 k_scan_fwd_chunk(int total, SSD_FWD_CHUNK_PARAMS) {
   if (S32 || !fast) {
     scan_fwd_chunk_block<PT, NT, NB, S32>(blockIdx.x, SSD_FWD_CHUNK_ARGS);

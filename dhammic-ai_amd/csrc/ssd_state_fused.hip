@@ -62,6 +62,10 @@ struct StateCfg {
   static size_t bytes(bool) { return (size_t)R * SLOT + (size_t)NW * TILE; }
   // waves per SIMD a block brings (its compute waves and one DMA wave per SIMD), at least two
   static constexpr int WPE = (NW + NPW + 3) / 4 > 2 ? (NW + NPW + 3) / 4 : 2;
+  // ... and at most: two blocks per CU of a two-wave block where their LDS fits. (With WPE as the limit the register
+  // allocation was padded until one block filled a CU: 128 one-token sequences of 16 heads of 128 columns, 4096 walks
+  // over 64 state columns, 74 -> 43 us.)
+  static constexpr int WPX = 2 * (R * SLOT + NW * TILE) <= 160 * 1024 && WPE == 2 ? 4 : WPE;
 };
 
 // Whether the walk uses the 64 x 16 wave tiles: the forward walk at PT = 2. The backward walk
@@ -394,9 +398,9 @@ __device__ __forceinline__ void state_step(const StateCtx& x, const unsigned cha
   cursor_step<FWD>(x, uc);
 }
 
-// StateCfg::WPE waves per SIMD: the block's compute and DMA waves (one block per CU at config sizes)
+// StateCfg::WPE to WPX waves per SIMD: the block's compute and DMA waves, once or twice
 template <int PT, int NT, bool FWD>
-__global__ void __launch_bounds__((StateCfg<PT, NT>::NTHR)) __attribute__((amdgpu_waves_per_eu(StateCfg<PT, NT>::WPE, StateCfg<PT, NT>::WPE)))
+__global__ void __launch_bounds__((StateCfg<PT, NT>::NTHR)) __attribute__((amdgpu_waves_per_eu(StateCfg<PT, NT>::WPE, StateCfg<PT, NT>::WPX)))
 k_state_fused(SsdDims d, const ChunkInfo* __restrict__ chunks,
                                                          const int32_t* __restrict__ seq_chunk0,
                                                          const int32_t* __restrict__ seq_order,

@@ -28,6 +28,25 @@ def _notes(elf):
             pos = data + (dlen + 3) // 4 * 4
 
 
+def _allocated_vgprs(elf):
+    """{kernel: VGPRs a wave is given} from the kernel descriptors (<kernel>.kd, 64 bytes; the low six bits of the
+    32-bit word at 48 count eights, less one): what decides the waves per SIMD, also where the compiler rounds the
+    allocation up to keep to a limit on them."""
+    shoff, = struct.unpack_from("<Q", elf, 40)
+    shentsize, shnum = struct.unpack_from("<HH", elf, 58)
+    sec = [struct.unpack_from("<IIQQQQIIQQ", elf, shoff + i * shentsize) for i in range(shnum)]
+    for _, kind, _, _, off, size, link, _, _, entsize in sec:
+        if kind != 11:  # SHT_DYNSYM
+            continue
+        names = sec[link][4]
+        for p in range(off, off + size, entsize):
+            st_name, _, _, shndx, value, _ = struct.unpack_from("<IBBHQQ", elf, p)
+            name = elf[names + st_name:elf.index(b"\0", names + st_name)].decode()
+            if name.endswith(".kd"):
+                at = sec[shndx][4] + value - sec[shndx][3]
+                yield name[:-3], ((struct.unpack_from("<I", elf, at + 48)[0] & 63) + 1) * 8
+
+
 @pytest.fixture(scope="module")
 def kernels_meta():
     from kernels import _capi
@@ -41,8 +60,11 @@ def kernels_meta():
             target = blob[pos + 24:pos + 24 + idlen]
             pos += 24 + idlen
             if b"gfx950" in target and size:
-                for note in _notes(blob[m.start() + off:m.start() + off + size]):
+                elf = blob[m.start() + off:m.start() + off + size]
+                for note in _notes(elf):
                     found.update({k[".name"]: k for k in note["amdhsa.kernels"]})
+                for name, n in _allocated_vgprs(elf):
+                    found[name]["allocated"] = n
     assert len(found) > 100
     return found
 
@@ -65,4 +87,16 @@ def test_row_kernel_leaves_room_for_two_blocks(kernels_meta):
         assert k[".vgpr_spill_count"] == 0, (pt, nt)
         ring = 3 * (2 * 2 * (32 * pt * 32 * nt + 64 * 32 * pt) + 1024)
         if nt <= 2 and 2 * (ring + 256) <= 160 * 1024:
-            assert k[".vgpr_count"] <= 128, (pt, nt, k[".vgpr_count"])
+            assert k["allocated"] <= 128, (pt, nt, k["allocated"])
+
+
+def test_walks_and_pair_scan_leave_room_for_two_blocks(kernels_meta):
+    """State walks of up to eight waves (2 per SIMD): at most 128 VGPRs, two blocks to a CU. The exact forward scan of
+    the halves of wide heads, one wave per SIMD: at most 256 for chunks of 64 and 128 tokens (for 128 with NT = 4 its
+    accumulators and S take more)."""
+    for (pt, nt, _), k in _variants(kernels_meta, "k_state_fused").items():
+        if pt * nt <= 4:
+            assert k["allocated"] <= 128, (pt, nt, k["allocated"])
+    for (pt, nt, nb, s32), k in _variants(kernels_meta, "k_scan_fwd_chunk").items():
+        if s32 and (nb == 1 or nb == 2 and nt < 4):
+            assert k["allocated"] <= 256, (pt, nt, nb, k["allocated"])
