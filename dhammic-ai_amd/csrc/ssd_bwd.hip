@@ -26,7 +26,8 @@ __device__ __forceinline__ void ld_per(const float* __restrict__ p, float (&o)[P
   }
 }
 
-template <typename T, int PER>
+// HS: two kernel heads per caller head (d.hs).
+template <typename T, int PER, bool HS>
 __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const ChunkInfo* __restrict__ chunks,
                                                     const float* __restrict__ Ah, const float* __restrict__ dt,
                                                     float* __restrict__ ddt, T* __restrict__ dA_tok,
@@ -35,14 +36,13 @@ __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const
   // thread t moves position t's four values with one 16-byte access through LDS (the per-head
   // 4-byte accesses touch a line per lane, four times as many L2 requests)
   __shared__ float s_dt[4][256], s_ddt[4][256];
-  // Two kernel heads per caller head (d.hs): the block's four heads are two caller heads, whose ddt and
-  // per-token da are summed through LDS; a wave past the last head repeats it (same values, no output of
-  // its own), so that every wave meets the barriers.
-  __shared__ float s_da[4][256];
+  // HS: the block's four heads are two caller heads, whose ddt and per-token da are summed through LDS; a
+  // wave past the last head repeats it (same values, no output of its own), so that every wave meets the
+  // barriers.
+  __shared__ float s_da[HS ? 4 : 1][HS ? 256 : 1];
   const int c = blockIdx.x;
   const int w = threadIdx.x >> 6;
-  const int hs = d.hs;
-  const int h = hs ? min((int)blockIdx.y * 4 + w, d.H - 1) : blockIdx.y * 4 + w;
+  const int h = HS ? min((int)blockIdx.y * 4 + w, d.H - 1) : blockIdx.y * 4 + w;
   const int lane = lane_id();
   if (h >= d.H) return;  // never taken when H % 4 == 0 (every wave of the block then has a head)
   const ChunkInfo ci = chunks[c];
@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const
     return;
   }
   const bool vec_dt = d.a_mode == 0 && d.has_dt && (d.H & 3) == 0 && (reinterpret_cast<uintptr_t>(dt) & 15) == 0;
-  const bool vec_ddt = !hs && vec_dt && ddt != nullptr && (reinterpret_cast<uintptr_t>(ddt) & 15) == 0;
+  const bool vec_ddt = !HS && vec_dt && ddt != nullptr && (reinterpret_cast<uintptr_t>(ddt) & 15) == 0;
   if (vec_dt) {
     const int tp = threadIdx.x;  // position; Qpad <= 256 = blockDim.x
     floatx4 q = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -135,12 +135,12 @@ __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const
     const int64_t row = ci.row0 + l;
     if (d.a_mode == 0) {
       const float dtv = vec_dt ? s_dt[w][l] : (d.has_dt ? dt[row * d.H + h] : 1.0f);
-      if (vec_ddt || hs) s_ddt[w][l] = (ddt && d.has_dt) ? t[e] + Ah[h >> hs] * da : 0.0f;
+      if (vec_ddt || HS) s_ddt[w][l] = (ddt && d.has_dt) ? t[e] + Ah[HS ? h >> 1 : h] * da : 0.0f;
       else if (ddt && d.has_dt) ddt[row * d.H + h] = t[e] + Ah[h] * da;
       dAp += dtv * da;
     } else {
       // per-token decay (with dt: the trapezoidal mode's scan, where a does not depend on dt)
-      if (hs) {
+      if constexpr (HS) {
         s_da[w][l] = da;
         s_ddt[w][l] = (ddt && d.has_dt) ? t[e] : 0.0f;
         continue;
@@ -152,7 +152,7 @@ __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const
   }
   for (int o = 32; o > 0; o >>= 1) dAp += __shfl_xor(dAp, o, 64);
   if (lane == 0) bf.dA_part[ch] = dAp;
-  if (hs) {
+  if constexpr (HS) {
     __syncthreads();
     const int tp = threadIdx.x, Hr = d.H >> 1;
     for (int q = 0; q < 2; ++q) {
@@ -201,11 +201,14 @@ size_t lds_bwd_row(int dtype, const SsdDims& d) {
 template <int PER>
 static void bwd_finish_launch(int dtype, dim3 grid, const SsdDims& d, const SsdBufs& b, const float* Ah,
                               const float* dt, float* ddt, void* dA_tok, float* da32, hipStream_t s) {
-  if (dtype == 1)
-    hipLaunchKernelGGL((k_bwd_finish<bf16, PER>), grid, dim3(256), 0, s, d, b, b.chunks, Ah, dt, ddt,
+  if (d.hs)  // (bf16 only)
+    hipLaunchKernelGGL((k_bwd_finish<bf16, PER, true>), grid, dim3(256), 0, s, d, b, b.chunks, Ah, dt, ddt,
+                       reinterpret_cast<bf16*>(dA_tok), da32);
+  else if (dtype == 1)
+    hipLaunchKernelGGL((k_bwd_finish<bf16, PER, false>), grid, dim3(256), 0, s, d, b, b.chunks, Ah, dt, ddt,
                        reinterpret_cast<bf16*>(dA_tok), da32);
   else
-    hipLaunchKernelGGL((k_bwd_finish<float, PER>), grid, dim3(256), 0, s, d, b, b.chunks, Ah, dt, ddt,
+    hipLaunchKernelGGL((k_bwd_finish<float, PER, false>), grid, dim3(256), 0, s, d, b, b.chunks, Ah, dt, ddt,
                        reinterpret_cast<float*>(dA_tok), da32);
 }
 
