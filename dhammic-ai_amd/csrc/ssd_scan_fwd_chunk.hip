@@ -28,6 +28,8 @@
 // Price, forward and backward at B=4 L=2048 H=16 P=128 N=64 chunk 256 with the norm: 254 -> 288 us (whole heads on
 // the general kernels: 605). Up to 128-token chunks two blocks share a CU, where a lone one waits for its loads: 8 x 2048
 // tokens of 32 heads of 128 columns, 32 groups, N=16, chunk 64, the forward 355 -> 249 us (whole heads 285).
+#include <stdint.h>
+
 #include <algorithm>
 
 #include "ssd_launch.h"
@@ -322,7 +324,19 @@ static hipError_t scan_fwd_chunk_t(const SsdDims& d, const SsdBufs& b, const Ssd
   if (ns < 1) ns = 1;
   if (ns > d.hpg) ns = d.hpg;
   int hslice = (d.hpg + ns - 1) / ns;
-  if (S32 && hslice < 2) hslice = 2;  // the halves of a head share S
+  if constexpr (S32) {
+    // the whole grid runs, each block building S for its heads: the slices whose blocks take the least time in passes
+    // over the chip, S at about two heads' time. The halves of a head share S.
+    const int slots = NB <= 2 ? 512 : 256;
+    int64_t best = INT64_MAX;
+    for (int q = 2; q <= std::max(2, d.hpg); ++q) {
+      const int64_t blocks = (int64_t)per * ((d.hpg + q - 1) / q), cost = (blocks + slots - 1) / slots * (q + 2);
+      if (cost < best) {
+        best = cost;
+        hslice = q;
+      }
+    }
+  }
   ns = (d.hpg + hslice - 1) / hslice;
   const size_t lds = FwdLds<PT, NT>::bytes(NB);
   ensure_lds(k_scan_fwd_chunk<PT, NT, NB, S32>, lds);
