@@ -184,14 +184,15 @@ __global__ void __launch_bounds__(256) k_f32_cb(SsdDims d, F32Args a) {
 }
 
 // ---------------------------------------------------------------------------
-// Forward chunk scan, Y = M x + exp(cs) C h_in^T (+ D x): block (unit, head, 64-column half of P); wave w has
+// Forward chunk scan, Y = M x + exp(cs) C h_in^T (+ D x): block (unit, head, 32 PT columns of P); wave w has
 // the row tiles w and nl - 1 - w, whose 32 x 32 source tiles number nl + 1 together, so the waves of a block
-// are even. x sits in LDS (70 KB at chunk 256: two blocks per CU); M is built in registers from the S tile
-// (loaded one tile ahead) and is the A operand as it is.
+// are even. x sits in LDS (70 KB at chunk 256, PT = 2: two blocks per CU); M is built in registers from the S tile
+// (ready one tile ahead) and is the A operand as it is. In small batches (launch_f32_scan) a wave has one row tile
+// and PT = 1; the two waves of a SIMD then share nl + 1 source tiles.
 // ---------------------------------------------------------------------------
 template <int PT, int NT, bool SELF>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) k_f32_scan(SsdDims d, F32Args a,
-                                                                                                         float* __restrict__ y, int nph) {
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_f32_scan(SsdDims d, F32Args a, float* __restrict__ y, int nph) {
   constexpr int PP = 32 * PT, XP = PP + 4;
   extern __shared__ __align__(16) unsigned char smem[];
   const int Qpad = d.Qpad, nl = Qpad / 32, nsub = nsub_of(nl);
@@ -205,39 +206,60 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   float* xs = s_dt + Qpad;                       // [Qpad][XP]
   const int64_t brow = (int64_t)d.G * d.N, xrow = (int64_t)d.H * d.P;
   const float* csc = a.cs + ((int64_t)c * d.H + h) * Qpad;
+  const int lane = lane_id(), hh = lane >> 5, l32 = lane & 31, w = threadIdx.x >> 6;
+  const int nlv = (ci.len + 31) / 32;
+  // tiles ta < tb; with a wave for every tile (two waves of a SIMD: 4 apart) the first alone
+  const bool single = (int)blockDim.x == 64 * nl;
+  const int ta = single && w >= 4 ? nl + 3 - w : w, tb = nl - 1 - w;
+  const bool two = !single && tb < nlv;
+  const int la = 32 * ta + l32, lb = 32 * tb + l32;
+  const float Dh = d.has_D ? a.Dv[h] : 0.0f;
+  // The operands of the state term's first 16 columns (SELF: of all, and C's again for S, whose first B rows come with
+  // them) in flight through the staging
+  constexpr int KC = SELF ? 2 * NT : 1;
+  const float* hrow = a.hin + (((int64_t)c * d.H + h) * d.Ppad + p0 + l32) * d.Npad + 8 * hh;
+  const __amdgpu_buffer_rsrc_t ra = buf_rsrc(a.Cm + (int64_t)(ci.row0 + 32 * ta) * brow + (int64_t)g * d.N);
+  const __amdgpu_buffer_rsrc_t rb = buf_rsrc(a.Cm + (int64_t)(ci.row0 + (two ? 32 * tb : 0)) * brow + (int64_t)g * d.N);
+  Frag<float> ca[KC], cb[KC], fh[KC][PT], fb[KC];
+  auto load = [&](int k) {
+    row_frags(ca, ra, l32 * (int)brow, la < ci.len, k + 8 * hh, d.N, d.vec_bc);
+    row_frags(cb, rb, l32 * (int)brow, two && lb < ci.len, k + 8 * hh, d.N, d.vec_bc);
+#pragma unroll
+    for (int i = 0; i < KC; ++i)
+#pragma unroll
+      for (int t = 0; t < PT; ++t) fh[i][t] = ld_frag(hrow + (int64_t)(32 * t) * d.Npad + k + 16 * i);
+  };
+  auto load_B = [&](int st) {
+    const __amdgpu_buffer_rsrc_t r = buf_rsrc(a.Bm + (int64_t)(ci.row0 + 32 * st) * brow + (int64_t)g * d.N);
+    row_frags(fb, r, l32 * (int)brow, 32 * st + l32 < ci.len, 8 * hh, d.N, d.vec_bc);
+  };
+  load(0);
+  if constexpr (SELF) load_B(0);
   stage_scalars(d, ci, csc, a.dt, nullptr, nullptr, h, s_cs, s_dt, nullptr);
   stage_rows<PP>(xs, XP, a.x + (int64_t)ci.row0 * xrow + (int64_t)h * d.P + p0, xrow, Qpad, ci.len, pw, d.vec_x);
   __syncthreads();
-  const int lane = lane_id(), hh = lane >> 5, l32 = lane & 31, w = threadIdx.x >> 6;
-  const int nlv = (ci.len + 31) / 32;
-  const int ta = w, tb = nl - 1 - w;  // ta < tb
   if (ta >= nlv) return;
-  const bool two = tb < nlv;
   floatx16 acc[2][PT];
 #pragma unroll
   for (int q = 0; q < 2; ++q)
 #pragma unroll
     for (int t = 0; t < PT; ++t) zero(acc[q][t]);
-  const int la = 32 * ta + l32, lb = 32 * tb + l32;
-  {
-    // operands of the next 16 columns in flight while these are multiplied
-    const float* hrow = a.hin + (((int64_t)c * d.H + h) * d.Ppad + p0 + l32) * d.Npad + 8 * hh;
-    const __amdgpu_buffer_rsrc_t ra = buf_rsrc(a.Cm + (int64_t)(ci.row0 + 32 * ta) * brow + (int64_t)g * d.N);
-    const __amdgpu_buffer_rsrc_t rb = buf_rsrc(a.Cm + (int64_t)(ci.row0 + (two ? 32 * tb : 0)) * brow + (int64_t)g * d.N);
-    Frag<float> ca[1], cb[1], fh[PT];
-    auto load = [&](int k) {
-      row_frags(ca, ra, l32 * (int)brow, la < ci.len, k + 8 * hh, d.N, d.vec_bc);
-      row_frags(cb, rb, l32 * (int)brow, two && lb < ci.len, k + 8 * hh, d.N, d.vec_bc);
+  if constexpr (SELF) {
 #pragma unroll
-      for (int t = 0; t < PT; ++t) fh[t] = ld_frag(hrow + (int64_t)(32 * t) * d.Npad + k);
-    };
-    load(0);
+    for (int k = 0; k < KC; ++k)
+#pragma unroll
+      for (int t = 0; t < PT; ++t) {
+        mma(acc[0][t], ca[k], fh[k][t]);
+        if (two) mma(acc[1][t], cb[k], fh[k][t]);
+      }
+  } else {
+    // operands of the next 16 columns in flight while these are multiplied
 #pragma unroll
     for (int k = 0; k < 32 * NT; k += 16) {
       const Frag<float> ca0 = ca[0], cb0 = cb[0];
       Frag<float> fh0[PT];
 #pragma unroll
-      for (int t = 0; t < PT; ++t) fh0[t] = fh[t];
+      for (int t = 0; t < PT; ++t) fh0[t] = fh[0][t];
       if (k + 16 < 32 * NT) load(k + 16);
 #pragma unroll
       for (int t = 0; t < PT; ++t) {
@@ -262,27 +284,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const float cs_a = s_cs[la], cs_b = s_cs[lb];
   const int strict = d.trapz ? 1 : 0;  // trapezoidal mode: strictly causal
   const int last = two ? tb : ta;
-  // S of the next source tile, ahead of its use: from memory, or (SELF) multiplied here
+  // S of the next source tile, ahead of its use: from memory, or (SELF) multiplied here, the B rows of the tile after
+  // it in flight
   floatx16 Sa, Sb;
-  Frag<float> ca[SELF ? 2 * NT : 1], cb[SELF ? 2 * NT : 1];
-  if constexpr (SELF) {
-    const __amdgpu_buffer_rsrc_t ra = buf_rsrc(a.Cm + (int64_t)(ci.row0 + 32 * ta) * brow + (int64_t)g * d.N);
-    const __amdgpu_buffer_rsrc_t rb = buf_rsrc(a.Cm + (int64_t)(ci.row0 + (two ? 32 * tb : 0)) * brow + (int64_t)g * d.N);
-    row_frags(ca, ra, l32 * (int)brow, la < ci.len, 8 * hh, d.N, d.vec_bc);
-    row_frags(cb, rb, l32 * (int)brow, two && lb < ci.len, 8 * hh, d.N, d.vec_bc);
-  }
   auto load_S = [&](int st, floatx16& A, floatx16& Bt) {
     if constexpr (SELF) {
-      const __amdgpu_buffer_rsrc_t r = buf_rsrc(a.Bm + (int64_t)(ci.row0 + 32 * st) * brow + (int64_t)g * d.N);
-      Frag<float> fb[SELF ? 2 * NT : 1];
-      row_frags(fb, r, l32 * (int)brow, 32 * st + l32 < ci.len, 8 * hh, d.N, d.vec_bc);
       zero(A);
       zero(Bt);
 #pragma unroll
-      for (int k = 0; k < 2 * NT; ++k) {
+      for (int k = 0; k < KC; ++k) {
         if (st <= ta) mma(A, fb[k], ca[k]);
         if (two) mma(Bt, fb[k], cb[k]);
       }
+      if (st < last) load_B(st + 1);
     } else {
       if (st <= ta) A = ld_tile(cbu + (int64_t)sub_of(ta, st) * 1024, lane);
       if (two) Bt = ld_tile(cbu + (int64_t)sub_of(tb, st) * 1024, lane);
@@ -291,7 +305,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   load_S(0, Sa, Sb);
   for (int st = 0; st <= last; ++st) {
     floatx16 Na, Nb;
-    if (st < last) load_S(st + 1, Na, Nb);
+    if (!SELF && st < last) load_S(st + 1, Na, Nb);
     float css[16], dts[16];
     rows16(s_cs + 32 * st, css);
     rows16(s_dt + 32 * st, dts);
@@ -322,10 +336,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int t = 0; t < PT; ++t) mfma32(acc[0][t], Sa[v], xv[t][v]);
     }
-    Sa = Na;
-    Sb = Nb;
+    if constexpr (SELF) {
+      if (st < last) load_S(st + 1, Sa, Sb);
+    } else {
+      Sa = Na;
+      Sb = Nb;
+    }
   }
-  const float Dh = d.has_D ? a.Dv[h] : 0.0f;
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     if (q == 1 && !two) continue;
@@ -352,14 +369,32 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 // row-major with the contraction along the rows, so every MFMA operand is one coalesced 4-byte load per lane
 // and nothing goes through LDS but the coefficients. One wave per 32 x 32 tile of the state.
 // ---------------------------------------------------------------------------
-template <int MODE>
+// STEP: tokens a step.
+template <int MODE, int STEP>
 __global__ void __launch_bounds__(512) k_f32_state(SsdDims d, F32Args a, const float* __restrict__ U,
                                                    const float* __restrict__ V, float* __restrict__ out) {
-  constexpr int NW = 1;
+  constexpr int NL = STEP / 2;  // loads per lane and operand
   __shared__ float coef[256];
   const int c = blockIdx.x, h = blockIdx.y, g = h / d.hpg;
   const ChunkInfo ci = a.chunks[c];
   if (ci.len == 0) return;
+  const int lane = lane_id(), hh = lane >> 5, l32 = lane & 31, w = threadIdx.x >> 6;  // one wave per tile
+  const int ntn = d.Npad / 32, pt = w / ntn, n0 = w % ntn * 32, p = 32 * pt + l32, n = n0 + l32;
+  const int64_t urow = (int64_t)d.H * d.P, vrow = (int64_t)d.G * d.N;
+  // a step's operands one step ahead; masked buffer loads (no branches) from bases at the step's first row
+  float uv[NL], vv[NL];
+  auto load = [&](int l0) {
+    const __amdgpu_buffer_rsrc_t ru = buf_rsrc(U + (int64_t)(ci.row0 + l0) * urow + (int64_t)h * d.P);
+    const __amdgpu_buffer_rsrc_t rv = buf_rsrc(V + (int64_t)(ci.row0 + l0) * vrow + (int64_t)g * d.N);
+#pragma unroll
+    for (int t = 0; t < NL; ++t) {
+      const int l = 2 * t + hh;
+      const bool ok = l0 + l < ci.len;
+      uv[t] = buf_ldf(ru, (l * (int)urow + p) * 4, ok && p < d.P);
+      vv[t] = buf_ldf(rv, (l * (int)vrow + n) * 4, ok && n < d.N);
+    }
+  };
+  load(0);
   const float* csc = a.cs + ((int64_t)c * d.H + h) * d.Qpad;
   const float cs_last = csc[d.Qpad - 1];
   for (int l = threadIdx.x; l < d.Qpad; l += blockDim.x) {
@@ -373,57 +408,22 @@ __global__ void __launch_bounds__(512) k_f32_state(SsdDims d, F32Args a, const f
     coef[l] = v;
   }
   __syncthreads();
-  const int lane = lane_id(), hh = lane >> 5, l32 = lane & 31;
-  const int ntw = (d.Npad / 32 + NW - 1) / NW, ntask = d.Ppad / 32 * ntw;
-  const int64_t urow = (int64_t)d.H * d.P, vrow = (int64_t)d.G * d.N;
-  for (int task = threadIdx.x >> 6; task < ntask; task += blockDim.x >> 6) {
-    const int pt = task / ntw, n0 = task % ntw * 32 * NW;
-    const int p = 32 * pt + l32;
-    floatx16 acc[NW];
+  floatx16 acc;
+  zero(acc);
+  for (int l0 = 0; l0 < ci.len; l0 += STEP) {
+    float ua[NL], va[NL];
 #pragma unroll
-    for (int q = 0; q < NW; ++q) zero(acc[q]);
-    // 16 tokens' operands one step ahead; masked buffer loads (no branches) from bases at the step's first row
-    float uv[8], vv[NW][8];
-    auto load = [&](int l0) {
-      const __amdgpu_buffer_rsrc_t ru = buf_rsrc(U + (int64_t)(ci.row0 + l0) * urow + (int64_t)h * d.P);
-      const __amdgpu_buffer_rsrc_t rv = buf_rsrc(V + (int64_t)(ci.row0 + l0) * vrow + (int64_t)g * d.N);
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int l = 2 * t + hh;
-        const bool ok = l0 + l < ci.len;
-        uv[t] = buf_ldf(ru, (l * (int)urow + p) * 4, ok && p < d.P);
-#pragma unroll
-        for (int q = 0; q < NW; ++q) {
-          const int n = n0 + 32 * q + l32;
-          vv[q][t] = buf_ldf(rv, (l * (int)vrow + n) * 4, ok && n < d.N);
-        }
-      }
-    };
-    load(0);
-    for (int l0 = 0; l0 < ci.len; l0 += 16) {
-      float ua[8], va[NW][8];
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        ua[t] = uv[t];
-        const float cf = coef[l0 + 2 * t + hh];  // (0 past the chunk)
-#pragma unroll
-        for (int q = 0; q < NW; ++q) va[q][t] = vv[q][t] * cf;
-      }
-      if (l0 + 16 < ci.len) load(l0 + 16);
-#pragma unroll
-      for (int t = 0; t < 8; ++t)
-#pragma unroll
-        for (int q = 0; q < NW; ++q) mfma32(acc[q], ua[t], va[q][t]);
+    for (int t = 0; t < NL; ++t) {
+      ua[t] = uv[t];
+      va[t] = vv[t] * coef[l0 + 2 * t + hh];  // (0 past the chunk; Qpad is a multiple of 64)
     }
-    float* o = out + ((int64_t)c * d.H + h) * d.Ppad * d.Npad;
+    if (l0 + STEP < ci.len) load(l0 + STEP);
 #pragma unroll
-    for (int q = 0; q < NW; ++q) {
-      if (n0 + 32 * q >= d.Npad) continue;
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        o[(int64_t)(32 * pt + acc_row(v, lane)) * d.Npad + n0 + 32 * q + l32] = acc[q][v];
-    }
+    for (int t = 0; t < NL; ++t) mfma32(acc, ua[t], va[t]);
   }
+  float* o = out + ((int64_t)c * d.H + h) * d.Ppad * d.Npad;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) o[(int64_t)(32 * pt + acc_row(v, lane)) * d.Npad + n] = acc[v];
 }
 
 // ---------------------------------------------------------------------------
@@ -492,18 +492,24 @@ __global__ void __launch_bounds__(256, 2) k_f32_col(SsdDims d, SsdBufs bf, F32Ar
       const float cs_s = s_cs[s_me], dt_s = s_dt[s_me];
       float gcol = 0.0f;
       floatx16 S;
-      Frag<float> bs[SELF ? 2 * NT : 1];
+      // (AHEAD: the C rows of the tile after the next are in flight; with PT = 4 they would spill)
+      constexpr bool AHEAD = SELF && PT <= 2;
+      Frag<float> bs[SELF ? 2 * NT : 1], fc[SELF ? 2 * NT : 1];
+      auto load_C = [&](int lt) {
+        row_frags(fc, buf_rsrc(a.Cm + (int64_t)(ci.row0 + 32 * lt) * brow + (int64_t)g * d.N), l32 * (int)brow,
+                  32 * lt + l32 < ci.len, 8 * hh, d.N, d.vec_bc);
+      };
       if constexpr (SELF)
         row_frags(bs, buf_rsrc(a.Bm + (int64_t)(ci.row0 + st_row) * brow + (int64_t)g * d.N), l32 * (int)brow,
                   s_me < ci.len, 8 * hh, d.N, d.vec_bc);
+      if constexpr (AHEAD) load_C(st);
       auto load_S = [&](int lt, floatx16& o) {
         if constexpr (SELF) {
-          Frag<float> fc[SELF ? 2 * NT : 1];
-          row_frags(fc, buf_rsrc(a.Cm + (int64_t)(ci.row0 + 32 * lt) * brow + (int64_t)g * d.N), l32 * (int)brow,
-                    32 * lt + l32 < ci.len, 8 * hh, d.N, d.vec_bc);
+          if constexpr (!AHEAD) load_C(lt);
           zero(o);
 #pragma unroll
           for (int k = 0; k < 2 * NT; ++k) mma(o, fc[k], bs[k]);
+          if (AHEAD && lt + 1 < nlv) load_C(lt + 1);
         } else {
           o = ld_tile(cbu + (int64_t)sub_of(lt, st) * 1024, lane);
         }
@@ -512,7 +518,7 @@ __global__ void __launch_bounds__(256, 2) k_f32_col(SsdDims d, SsdBufs bf, F32Ar
       for (int lt = st; lt < nlv; ++lt) {
         floatx16 nS;
         const int64_t so = (int64_t)sub_of(lt, st) * 1024;
-        if (lt + 1 < nlv) load_S(lt + 1, nS);
+        if (!AHEAD && lt + 1 < nlv) load_S(lt + 1, nS);
         Frag<float> yf[PP / 16];
 #pragma unroll
         for (int k = 0; k < PP / 16; ++k) yf[k] = ld_frag(dys + (32 * lt + l32) * YP + 16 * k + 8 * hh);
@@ -561,7 +567,11 @@ __global__ void __launch_bounds__(256, 2) k_f32_col(SsdDims d, SsdBufs bf, F32Ar
 #pragma unroll
           for (int v = 0; v < 16; ++v) mfma32(dX[t], S[v], yv[t & 1][v]);
         }
-        S = nS;
+        if constexpr (AHEAD) {
+          if (lt + 1 < nlv) load_S(lt + 1, S);
+        } else {
+          S = nS;
+        }
       }
       gcol = add_xor32(gcol);
       if (hh == 0 && s_me < ci.len) bf.colG[hq + s_me] = gcol;
@@ -868,11 +878,12 @@ static void cb_launch(const SsdDims& d, const F32Args& a, int units, hipStream_t
 // head would read the tiles, and a launch and their way through memory are saved).
 static bool f32_self(const SsdDims& d) { return d.hpg == 1 && d.Npad == 32; }
 
+// `few`: a wave per tile.
 template <int PT, int NT>
-static hipError_t f32_scan_t(const SsdDims& d, const SsdBufs& b, F32Args a, float* y, hipStream_t s) {
-  const int units = d.max_chunks * d.G, nph = d.Ppad / (32 * PT);
+static hipError_t f32_scan_t(const SsdDims& d, const SsdBufs& b, F32Args a, float* y, bool few, hipStream_t s) {
+  const int units = d.max_chunks * d.G, nph = (d.P + 32 * PT - 1) / (32 * PT), nl = d.Qpad / 32;
   const size_t lds = sizeof(float) * ((size_t)2 * d.Qpad + (size_t)d.Qpad * (32 * PT + 4));
-  const dim3 thr(64 * ((d.Qpad / 32 + 1) / 2));
+  const dim3 thr(64 * (few ? nl : (nl + 1) / 2));
   if (f32_self(d)) {
     ensure_lds(k_f32_scan<PT, NT, NT == 1>, lds);
     hipLaunchKernelGGL((k_f32_scan<PT, NT, NT == 1>), dim3((unsigned)units * nph), thr, lds, s, d, a, y, nph);
@@ -891,13 +902,18 @@ static hipError_t f32_scan_t(const SsdDims& d, const SsdBufs& b, F32Args a, floa
 hipError_t launch_f32_scan(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s) {
   const F32Args a = f32_args(b, in, nullptr);
   float* yo = static_cast<float*>(y);
-  switch ((d.Ppad > 32 ? 20 : 10) + d.Npad / 32) {
-    case 11: return f32_scan_t<1, 1>(d, b, a, yo, s);
-    case 12: return f32_scan_t<1, 2>(d, b, a, yo, s);
-    case 14: return f32_scan_t<1, 4>(d, b, a, yo, s);
-    case 21: return f32_scan_t<2, 1>(d, b, a, yo, s);
-    case 22: return f32_scan_t<2, 2>(d, b, a, yo, s);
-    default: return f32_scan_t<2, 4>(d, b, a, yo, s);
+  // A wave per tile over 32 columns of P where those waves, two per SIMD, fit the chip at once: the scan is then one
+  // wave's chain of products, half as long. Forward alone, two tiles of 64 columns / one of 32, us: 32 chunks of 64
+  // tokens, 4 heads of 64 columns 50 / 37; 8 chunks of 64, 24 heads of 96 47 / 36; 128 chunk-heads of 256 tokens (2048
+  // waves) 66 / 55; 512 of them 96 / 146.
+  const bool few = (int64_t)d.max_chunks * d.H * ((d.P + 31) / 32) * (d.Qpad / 32) <= 2048;
+  switch ((d.P > 32 && !few ? 20 : 10) + d.Npad / 32) {
+    case 11: return f32_scan_t<1, 1>(d, b, a, yo, few, s);
+    case 12: return f32_scan_t<1, 2>(d, b, a, yo, few, s);
+    case 14: return f32_scan_t<1, 4>(d, b, a, yo, few, s);
+    case 21: return f32_scan_t<2, 1>(d, b, a, yo, few, s);
+    case 22: return f32_scan_t<2, 2>(d, b, a, yo, few, s);
+    default: return f32_scan_t<2, 4>(d, b, a, yo, few, s);
   }
 }
 
@@ -908,9 +924,13 @@ hipError_t launch_f32_state(int mode, const SsdDims& d, const SsdBufs& b, const 
   const F32Args a = f32_args(b, in, nullptr);
   const dim3 grid(d.max_chunks, d.H);
   const float *u = static_cast<const float*>(U), *v = static_cast<const float*>(V);
-  const dim3 thr(64 * min(8, d.Ppad / 32 * (d.Npad / 32)));
-  if (mode == 0) hipLaunchKernelGGL(k_f32_state<0>, grid, thr, 0, s, d, a, u, v, out);
-  else hipLaunchKernelGGL(k_f32_state<1>, grid, thr, 0, s, d, a, u, v, out);
+  const dim3 thr(64 * (d.Ppad / 32) * (d.Npad / 32));  // (at most 8 tiles: not 128 x 128)
+  // Up to two waves per SIMD wait for their loads, so they take twice as many at once (48 states of 32 x 16 over 256
+  // tokens 13.7 -> 12.1 us); more hide each other's, and short chunks would multiply padding (1536 states of 64 x 128
+  // over one token: 6 us dearer with steps of 32).
+  const bool few = (int64_t)d.max_chunks * d.H * (thr.x / 64) <= 2048 && d.Qpad > 64;
+  auto k = mode == 0 ? (few ? k_f32_state<0, 32> : k_f32_state<0, 16>) : (few ? k_f32_state<1, 32> : k_f32_state<1, 16>);
+  hipLaunchKernelGGL(k, grid, thr, 0, s, d, a, u, v, out);
   return hipGetLastError();
 }
 

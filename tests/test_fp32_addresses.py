@@ -21,7 +21,7 @@ int main() {
   long pieces = 0;
   const int64_t strides[] = {65535LL * 128, 36500LL * 128, 33};
   for (int W : {32, 64, 128})
-    for (int nthr : {64, 128, 192, 256})
+    for (int nthr : {64, 128, 192, 256, 384, 512})
       for (int64_t ld : strides) {
         const int cpr = W / 4, total = 256 * cpr, NB = 8;
         bool seen[256 * 32] = {};

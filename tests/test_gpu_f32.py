@@ -106,3 +106,30 @@ def test_halves_of_wide_heads_at_the_largest_row_strides():
                                             A[lo:lo + k].contiguous(), B, C, 256)
             assert torch.equal(y[:, :, lo:lo + k], got)
             assert y[:, 115:, lo:lo + k].abs().min() > 0
+
+
+@pytest.mark.parametrize("off", [False, True], ids=["aligned", "unaligned"])
+@pytest.mark.parametrize("P,H,G,N,Q,L", [
+    (32, 4, 1, 16, 64, 65), (33, 3, 3, 31, 64, 100), (64, 4, 4, 33, 128, 257), (64, 6, 2, 128, 192, 383),
+    (128, 2, 1, 64, 256, 300), (100, 2, 2, 20, 256, 513), (64, 3, 3, 32, 256, 256), (20, 2, 2, 12, 256, 31)])
+def test_small_batches_are_the_same_bits(P, H, G, N, Q, L, off):
+    """The scan's two splits (a wave per tile over 32 columns up to 2048 such waves, two tiles over 64 columns past
+    them) and the states' two step lengths make the same sums: a batch past the rule against its first and last
+    sequences alone."""
+    import kernels
+    per = -(-L // Q) * H * -(-P // 32) * (-(-Q // 64) * 2)
+    b = 2048 // per + 1
+    assert per <= 2048 < b * per
+    inp = {k: v.to(DEV) for k, v in make_inputs(SsdShape(b, L, H, P, G, N, Q), seed=P, with_init=True).items()}
+    place = (lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)) if off else (lambda t: t.contiguous())
+
+    def run(lo, hi):
+        x, dt, B, C, init = (place(inp[k][lo:hi]) for k in ("x", "dt", "B", "C", "init"))
+        with torch.no_grad():
+            return kernels.ssd_scan_combined(x, dt, inp["A"], B, C, Q, D=inp["D"], initial_states=init,
+                                             return_final_state=True)
+
+    y, fin = run(0, b)
+    for i in (0, b - 1):
+        yi, fi = run(i, i + 1)
+        assert torch.equal(y[i:i + 1], yi) and torch.equal(fin[i:i + 1], fi)
