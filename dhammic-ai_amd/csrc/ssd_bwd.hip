@@ -1,5 +1,5 @@
-// Backward of the chunked SSD scan: the finish kernel, and the LDS sizes of the column / row kernels
-// (ssd_bwd_impl.h), which bound the shapes the C ABI takes.
+// Backward of the chunked SSD scan: the finish kernel, and the LDS sizes of the general bf16 column / row kernels
+// (ssd_bwd_impl.h).
 #include "ssd_launch.h"
 
 // ---------------------------------------------------------------------------
@@ -179,8 +179,8 @@ __global__ void __launch_bounds__(256) k_bwd_finish(SsdDims d, SsdBufs bf, const
   }
 }
 
-size_t lds_bwd_col(int dtype, const SsdDims& d) {
-  const size_t es = dtype == 1 ? 2 : 4;
+size_t lds_bwd_col(const SsdDims& d) {
+  const size_t es = 2;
   const size_t NP = d.Npad + 16 / es, PP = d.Ppad + 16 / es, BP = SSD_BLK + 16 / es;
   const size_t tiles = (d.Ppad > d.Npad ? d.Ppad : d.Npad) / 32;
   const size_t fixed = sizeof(float) * (2 * d.Qpad + 4 * SSD_BLK) + es * (SSD_BLK * NP + SSD_BLK * PP);
@@ -189,8 +189,8 @@ size_t lds_bwd_col(int dtype, const SsdDims& d) {
   return fixed + (regA > regB ? regA : regB);
 }
 
-size_t lds_bwd_row(int dtype, const SsdDims& d) {
-  const size_t es = dtype == 1 ? 2 : 4;
+size_t lds_bwd_row(const SsdDims& d) {
+  const size_t es = 2;
   const size_t NP = d.Npad + 16 / es, PP = d.Ppad + 16 / es, BP = SSD_BLK + 16 / es;
   const size_t fixed = sizeof(float) * (2 * d.Qpad + 4 * SSD_BLK) + es * (SSD_BLK * NP + SSD_BLK * PP);
   const size_t regA = es * (SSD_BLK * NP + SSD_BLK * PP + d.Npad * BP);

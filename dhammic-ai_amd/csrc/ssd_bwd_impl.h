@@ -20,8 +20,8 @@
 
 #include "ssd_launch.h"
 
-size_t lds_bwd_col(int dtype, const SsdDims& d);
-size_t lds_bwd_row(int dtype, const SsdDims& d);
+size_t lds_bwd_col(const SsdDims& d);
+size_t lds_bwd_row(const SsdDims& d);
 
 
 
@@ -474,7 +474,7 @@ template <typename T, int PT, int NT>
 hipError_t bwd_col_t(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dx, void* dB,
                             hipStream_t s) {
   dim3 grid(d.Qpad / SSD_BLK, d.G * b.nslices, d.max_chunks);
-  const size_t lds = lds_bwd_col(sizeof(T) == 2 ? 1 : 0, d);
+  const size_t lds = lds_bwd_col(d);
   ensure_lds(k_bwd_col<T, PT, NT>, lds);
   hipLaunchKernelGGL((k_bwd_col<T, PT, NT>), grid, dim3(256), lds, s, d, b, make_common<T>(d, b, in, dy),
                      reinterpret_cast<T*>(dx), reinterpret_cast<T*>(dB));
@@ -506,7 +506,7 @@ template <typename T, int PT, int NT>
 hipError_t bwd_row_t(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dC,
                             hipStream_t s) {
   dim3 grid(d.Qpad / SSD_BLK, d.G * b.nslices, d.max_chunks);
-  const size_t lds = lds_bwd_row(sizeof(T) == 2 ? 1 : 0, d);
+  const size_t lds = lds_bwd_row(d);
   ensure_lds(k_bwd_row<T, PT, NT>, lds);
   hipLaunchKernelGGL((k_bwd_row<T, PT, NT>), grid, dim3(256), lds, s, d, b, make_common<T>(d, b, in, dy),
                      reinterpret_cast<T*>(dC));

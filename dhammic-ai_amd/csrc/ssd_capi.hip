@@ -125,11 +125,14 @@ int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
   p->dtype = s->dtype;
   p->state_dtype = s->state_dtype;
   p->fused_bwd = bwd_main_supported(p->dtype, d) ? 1 : 0;
-  if ((scan_fwd_chunk_supported(p->dtype, d) ? std::max(lds_scan_fwd_chunk(d), lds_scan_fwd_fact(d))
-                                              : lds_chunk_scan_fwd(p->dtype, d)) > kMaxLds ||
-      (p->fused_bwd ? (lds_bwd_main(d) > kMaxLds || lds_bwd_fact(d) > kMaxLds || lds_bwd_gemm(d) > kMaxLds)
-                    : (lds_bwd_col(p->dtype, d) > kMaxLds || lds_bwd_row(p->dtype, d) > kMaxLds)))
+  if (p->dtype == SSD_DTYPE_F32) {
+    if (!f32_supported(d, kMaxLds)) return SSD_ERR_UNSUPPORTED;
+  } else if ((scan_fwd_chunk_supported(p->dtype, d) ? std::max(lds_scan_fwd_chunk(d), lds_scan_fwd_fact(d))
+                                                    : lds_chunk_scan_fwd(d)) > kMaxLds ||
+             (p->fused_bwd ? (lds_bwd_main(d) > kMaxLds || lds_bwd_fact(d) > kMaxLds || lds_bwd_gemm(d) > kMaxLds)
+                           : (lds_bwd_col(d) > kMaxLds || lds_bwd_row(d) > kMaxLds))) {
     return SSD_ERR_UNSUPPORTED;
+  }
 
   // head slices of the backward: enough blocks to fill the chip, fewest partials
   int64_t ns;

@@ -866,6 +866,23 @@ static F32Args f32_args(const SsdBufs& b, const SsdIn& in, const void* dy) {
   return a;
 }
 
+// LDS of the kernels, for PT (and NT) tiles of 32 columns
+static size_t lds_f32_scan(const SsdDims& d, int pt) {
+  return sizeof(float) * ((size_t)2 * d.Qpad + (size_t)d.Qpad * (32 * pt + 4));
+}
+static size_t lds_f32_col(const SsdDims& d, int pt) {
+  return sizeof(float) * ((size_t)3 * d.Qpad + 16 + (size_t)(d.Qpad / 32) * d.Qpad + (size_t)d.Qpad * (32 * pt + 4));
+}
+static size_t lds_f32_row(int pt, int nt) { return sizeof(float) * (1024 * pt * nt + 256); }
+
+// Widths of 32, 64 and 128 columns in any pairing but 128 x 128 (the switches below, and one wave per state tile
+// in k_f32_state).
+bool f32_supported(const SsdDims& d, size_t max_lds) {
+  const int pt = d.Ppad / 32, nt = d.Npad / 32;
+  return pt * nt <= 8 && d.Qpad <= 256 && lds_f32_scan(d, pt < 2 ? pt : 2) <= max_lds && lds_f32_col(d, pt) <= max_lds &&
+         lds_f32_row(pt, nt) <= max_lds;
+}
+
 size_t f32_unit_floats(const SsdDims& d) { return (size_t)nsub_of(d.Qpad / 32) * 1024; }
 
 template <int NT, bool FWD>
@@ -882,7 +899,7 @@ static bool f32_self(const SsdDims& d) { return d.hpg == 1 && d.Npad == 32; }
 template <int PT, int NT>
 static hipError_t f32_scan_t(const SsdDims& d, const SsdBufs& b, F32Args a, float* y, bool few, hipStream_t s) {
   const int units = d.max_chunks * d.G, nph = (d.P + 32 * PT - 1) / (32 * PT), nl = d.Qpad / 32;
-  const size_t lds = sizeof(float) * ((size_t)2 * d.Qpad + (size_t)d.Qpad * (32 * PT + 4));
+  const size_t lds = lds_f32_scan(d, PT);
   const dim3 thr(64 * (few ? nl : (nl + 1) / 2));
   if (f32_self(d)) {
     ensure_lds(k_f32_scan<PT, NT, NT == 1>, lds);
@@ -942,7 +959,7 @@ static hipError_t f32_bwd_t(const SsdDims& d, const SsdBufs& b, F32Args a, float
   const int64_t ss = (int64_t)b.f32_batch * f32_unit_floats(d);
   a.unit0 = u0;
   if (!row) {
-    const size_t lds = sizeof(float) * ((size_t)3 * d.Qpad + 16 + (size_t)nl * d.Qpad + (size_t)d.Qpad * (32 * PT + 4));
+    const size_t lds = lds_f32_col(d, PT);
     const int nhalf = nl >= 6 ? 2 : 1;
     const dim3 grid((unsigned)n * b.nslices * nhalf), thr(64 * min(nl, 4));
     if (f32_self(d)) {
@@ -957,7 +974,7 @@ static hipError_t f32_bwd_t(const SsdDims& d, const SsdBufs& b, F32Args a, float
     if (b.nslices > 1)
       hipLaunchKernelGGL(k_f32_ds, dim3((unsigned)n * ((nsub_of(nl) + 3) / 4)), dim3(256), 0, s, d, b.chunks, u0,
                          b.f32_dS, ss, b.nslices);
-    const size_t lds = sizeof(float) * (1024 * PT * NT + 256);
+    const size_t lds = lds_f32_row(PT, NT);
     hipLaunchKernelGGL((k_f32_row<PT, NT>), dim3((unsigned)n * 2 * ((nl + 3) / 4) * b.f32_rsl), dim3(NT > 2 ? 512 : 256), lds, s, d, b,
                        a, b.f32_dS, dB, dC, b.f32_rhs, b.f32_rsl > 1 ? b.f32_rsl - 1 : 1, b.f32_rsl);
   }
@@ -976,7 +993,8 @@ static hipError_t f32_bwd(const SsdDims& d, const SsdBufs& b, const SsdIn& in, c
     case 22: return f32_bwd_t<2, 2>(d, b, a, px, pb, pc, u0, n, row, s);
     case 24: return f32_bwd_t<2, 4>(d, b, a, px, pb, pc, u0, n, row, s);
     case 41: return f32_bwd_t<4, 1>(d, b, a, px, pb, pc, u0, n, row, s);
-    default: return f32_bwd_t<4, 2>(d, b, a, px, pb, pc, u0, n, row, s);
+    case 42: return f32_bwd_t<4, 2>(d, b, a, px, pb, pc, u0, n, row, s);
+    default: return hipErrorInvalidValue;  // (f32_supported)
   }
 }
 

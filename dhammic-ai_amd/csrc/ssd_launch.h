@@ -70,11 +70,12 @@ hipError_t launch_scan_fwd_fact(const SsdDims& d, const SsdBufs& b, const SsdIn&
 
 // ssd_scan_fwd.hip (bf16 shapes outside the fused path)
 hipError_t launch_chunk_scan_fwd(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s);
-size_t lds_chunk_scan_fwd(int dtype, const SsdDims& d);
+size_t lds_chunk_scan_fwd(const SsdDims& d);
 
 // ssd_f32.hip (fp32): the forward chunk scan, the chunk states (modes of launch_chunk_state), and the
 // backward of units [u0, u0 + n) (units: chunk * G + group), column side then row side
 size_t f32_unit_floats(const SsdDims& d);  // S (or dS) tiles of one unit
+bool f32_supported(const SsdDims& d, size_t max_lds);
 hipError_t launch_f32_scan(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s);
 hipError_t launch_f32_state(int mode, const SsdDims& d, const SsdBufs& b, const void* U, const void* V, const float* dt,
                             float* out, hipStream_t s);
@@ -91,8 +92,8 @@ hipError_t launch_bwd_row(const SsdDims& d, const SsdBufs& b, const SsdIn& in, c
 // ddt and da32 (fp32 per-token decay gradient, a_mode PER_TOKEN) are optional
 hipError_t launch_bwd_finish(int dtype, const SsdDims& d, const SsdBufs& b, const SsdIn& in,
                              float* ddt, void* dA_tok, float* da32, hipStream_t s);
-size_t lds_bwd_col(int dtype, const SsdDims& d);
-size_t lds_bwd_row(int dtype, const SsdDims& d);
+size_t lds_bwd_col(const SsdDims& d);
+size_t lds_bwd_row(const SsdDims& d);
 
 // Fixup launches (k_scan_fwd_chunk, k_bwd_main with the k_chunk_cumsum flags): at most this many units per
 // block of their chip-sized grid

@@ -153,8 +153,7 @@ inline size_t lds_scan_fwd_hs(size_t es, const SsdDims& d, size_t hs) {
 // one CU's LDS (80 KiB each), else 1. All heads of a block share B and C; two
 // heads keep the register count low enough for two blocks per CU, whose
 // interleaving hides the barrier and load latency of each.
-inline int fwd_heads_per_block(int dtype, const SsdDims& d) {
-  const size_t es = dtype == 1 ? 2 : 4;
+inline int fwd_heads_per_block(size_t es, const SsdDims& d) {
   if (d.hpg % 2 == 0 && lds_scan_fwd_hs(es, d, 2) <= 80 * 1024) return 2;
   return 1;
 }
@@ -191,7 +190,7 @@ hipError_t scan_fwd_p(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void*
 
 template <typename T>
 hipError_t scan_fwd_dispatch(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s) {
-  const int hs = fwd_heads_per_block(sizeof(T) == 2 ? 1 : 0, d);
+  const int hs = fwd_heads_per_block(sizeof(T), d);
   if (hs == 2) return scan_fwd_p<T, 2>(d, b, in, y, s);
   return scan_fwd_p<T, 1>(d, b, in, y, s);
 }

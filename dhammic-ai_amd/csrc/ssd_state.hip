@@ -79,8 +79,8 @@ __global__ void __launch_bounds__(256) k_chunk_state(SsdDims d, const ChunkInfo*
   }
 }
 
-static size_t lds_chunk_state(int dtype, const SsdDims& d) {
-  const size_t es = dtype == 1 ? 2 : 4;
+static size_t lds_chunk_state(const SsdDims& d) {
+  const size_t es = sizeof(bf16);
   const int KP = SSD_BLK + 16 / (int)es;
   return es * (size_t)(d.Ppad + d.Npad) * KP + sizeof(float) * d.Qpad;
 }
@@ -89,7 +89,7 @@ hipError_t launch_chunk_state(int dtype, int mode, const SsdDims& d, const SsdBu
                               const void* V, const float* dt, float* out, hipStream_t s) {
   if (dtype != 1) return launch_f32_state(mode, d, b, U, V, dt, out, s);
   dim3 grid(d.max_chunks, d.H);
-  const size_t lds = lds_chunk_state(dtype, d);
+  const size_t lds = lds_chunk_state(d);
   auto k = mode == 0 ? k_chunk_state<bf16, 0> : k_chunk_state<bf16, 1>;
   ensure_lds(k, lds);
   hipLaunchKernelGGL(k, grid, dim3(256), lds, s, d, b.chunks, b.cs, reinterpret_cast<const bf16*>(U),

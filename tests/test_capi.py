@@ -129,6 +129,15 @@ def test_validation_rejects(capi, kw, status):
     assert _validate(capi, **kw) == getattr(capi, status)
 
 
+@pytest.mark.parametrize("chunk", [1, 64, 65, 192, 256])
+def test_fp32_shapes(capi, chunk):
+    """The fp32 kernels take every pairing of 32, 64 and 128 padded columns but 128 x 128, whatever the chunk."""
+    for P in (1, 32, 33, 64, 65, 128):
+        for N in (1, 32, 33, 64, 65, 128):
+            want = capi.SSD_ERR_UNSUPPORTED if P > 64 and N > 64 else capi.SSD_OK
+            assert _validate(capi, dtype=capi.SSD_DTYPE_F32, headdim=P, dstate=N, chunk=chunk, has_z=0) == want, (P, N)
+
+
 def test_workspace_sizes(capi):
     lib = capi.load()
     d = _desc(capi)
