@@ -172,12 +172,14 @@ int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
   const int64_t units = max_chunks * d.G;
   const bool f32 = s->dtype == SSD_DTYPE_F32;
   const size_t unit_bytes = f32 ? f32_unit_floats(d) * sizeof(float) : 0;
+  const size_t s_bytes = f32 && !f32_self(d) ? unit_bytes : 0;  // S tiles of a unit
   if (f32) {
     constexpr int64_t kFwdTiles = 512ll << 20, kBwdTiles = 1ll << 30;
     const int64_t st_bytes = max_chunks * d.H * d.Ppad * d.Npad * 4;
-    const int64_t fb = (tight ? st_bytes : std::max(st_bytes, kFwdTiles)) / (int64_t)unit_bytes;
-    p->f32_fbatch = (int)std::max<int64_t>(1, std::min(units, fb));
-    p->f32_bbatch = (int)std::max<int64_t>(1, std::min(units, kBwdTiles / ((p->nslices + 1) * (int64_t)unit_bytes)));
+    const int64_t fb = s_bytes ? (tight ? st_bytes : std::max(st_bytes, kFwdTiles)) / (int64_t)s_bytes : units;
+    const int64_t bb = kBwdTiles / (int64_t)(p->nslices * unit_bytes + s_bytes);
+    p->f32_fbatch = (int)std::max<int64_t>(1, std::min({units, fb, (int64_t)INT32_MAX}));
+    p->f32_bbatch = (int)std::max<int64_t>(1, std::min(units, bb));
     int64_t nhs = 2048 / (units * 2 * (d.Qpad / 32)) - 1;
     nhs = std::min<int64_t>(std::max<int64_t>(nhs, 1), d.hpg);
     p->f32_rhs = (int)((d.hpg + nhs - 1) / nhs);
@@ -219,7 +221,7 @@ int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
   p->saved_bytes = off;
   off = 0;
   // (fp32: the scan's S tiles, once the chunk states have been used)
-  p->o_st = take(std::max(MC * H * PN * sizeof(float), p->f32_fbatch * unit_bytes));
+  p->o_st = take(std::max(MC * H * PN * sizeof(float), p->f32_fbatch * s_bytes));
   p->o_ffac = take(MC * H * d.Qpad * sizeof(float));
   p->o_ffac2 = d.trapz == SSD_TRAPZ_DROP_BETA_DA ? take(MC * H * d.Qpad * sizeof(float)) : 0;
   p->fwd_bytes = off;
@@ -239,7 +241,7 @@ int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
   const int64_t nparts = f32 ? p->f32_rsl : std::max<int64_t>(p->nslices, p->fused_bwd ? p->gemm_parts : 1);
   p->o_dBp = nparts > 1 ? take(nparts * bcn) : 0;
   p->o_dCp = nparts > 1 ? take(nparts * bcn) : 0;
-  p->o_bcb = f32 ? take(p->f32_bbatch * unit_bytes) : 0;
+  p->o_bcb = s_bytes ? take(p->f32_bbatch * s_bytes) : 0;
   p->o_fdS = f32 ? take(p->nslices * p->f32_bbatch * unit_bytes) : 0;
   const size_t nbq = (size_t)(d.Qpad / SSD_BLK);
   const bool tiles = p->fused_bwd;

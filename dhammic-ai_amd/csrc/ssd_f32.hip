@@ -893,7 +893,7 @@ static void cb_launch(const SsdDims& d, const F32Args& a, int units, hipStream_t
 
 // One head per group and N <= 32: the scan and the column kernel multiply S themselves (16 MFMA a tile; no other
 // head would read the tiles, and a launch and their way through memory are saved).
-static bool f32_self(const SsdDims& d) { return d.hpg == 1 && d.Npad == 32; }
+bool f32_self(const SsdDims& d) { return d.hpg == 1 && d.Npad == 32; }
 
 // `few`: a wave per tile.
 template <int PT, int NT>

@@ -76,6 +76,7 @@ size_t lds_chunk_scan_fwd(const SsdDims& d);
 // backward of units [u0, u0 + n) (units: chunk * G + group), column side then row side
 size_t f32_unit_floats(const SsdDims& d);  // S (or dS) tiles of one unit
 bool f32_supported(const SsdDims& d, size_t max_lds);
+bool f32_self(const SsdDims& d);  // S is multiplied where it is used: no tiles of it
 hipError_t launch_f32_scan(const SsdDims& d, const SsdBufs& b, const SsdIn& in, void* y, hipStream_t s);
 hipError_t launch_f32_state(int mode, const SsdDims& d, const SsdBufs& b, const void* U, const void* V, const float* dt,
                             float* out, hipStream_t s);

@@ -138,6 +138,20 @@ def test_fp32_shapes(capi, chunk):
             assert _validate(capi, dtype=capi.SSD_DTYPE_F32, headdim=P, dstate=N, chunk=chunk, has_z=0) == want, (P, N)
 
 
+def test_fp32_workspaces_hold_no_tiles_that_nothing_reads(capi):
+    """One head per group and N <= 32: S is multiplied in place, so the forward scratch is the chunk states and the
+    decay factors alone, and the backward has dS tiles but none of S."""
+    lib = capi.load()
+    size = lambda kind, **kw: lib.ssd_workspace_bytes(ctypes.byref(_desc(  # noqa: E731
+        capi, dtype=capi.SSD_DTYPE_F32, has_z=0, batch=8, seqlen=4096, nheads=32, headdim=32, **kw)), kind)
+    chunks, unit = 8 * 16 * 32, 36 * 4096
+    factors = chunks * 256 * 4
+    assert size(capi.SSD_WS_FWD_SCRATCH, ngroups=32, dstate=16) == chunks * 32 * 32 * 4 + factors
+    assert size(capi.SSD_WS_FWD_SCRATCH, ngroups=32, dstate=33) > 500 << 20  # (tiles, one batch)
+    grown = size(capi.SSD_WS_BWD_SCRATCH, ngroups=32, dstate=16) - chunks * 10 * 256 * 4
+    assert grown < chunks * unit + (64 << 20)
+
+
 def test_workspace_sizes(capi):
     lib = capi.load()
     d = _desc(capi)
