@@ -106,7 +106,12 @@ int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
   // A, B, C and D, so a wider one whose half is a whole number of 16-byte vectors runs as two kernel heads of
   // P / 2 that share them: x, y, z, the states and their gradients keep their layout (heads are the slower
   // dimension), the cumsum launch repeats dt and D, and the finish sums the gradients of the pair.
-  if (!tight && s->dtype == SSD_DTYPE_BF16 && d.P > 64 && d.P % 16 == 0 && d.N % 8 == 0 && 2 * s->nheads <= kMaxGrid) {
+  // Past two limits the head stays whole on the general kernels, whose grids have three axes and whose backward
+  // keeps no tiles of dS: the pairs' grids on one axis (at most 1024 threads per chunk and kernel head; a launch takes
+  // 2^32), and dS tiles of 16 GiB.
+  const int64_t nbk = round_up(d.Q, SSD_BLK) / SSD_BLK, pair_tiles = max_chunks * d.G * nbk * nbk * 4096 * 6;
+  if (!tight && s->dtype == SSD_DTYPE_BF16 && d.P > 64 && d.P % 16 == 0 && d.N % 8 == 0 && 2 * s->nheads <= kMaxGrid &&
+      max_chunks * s->nheads * 2 * 1024 <= (int64_t)UINT32_MAX && pair_tiles <= 16ll << 30) {
     d.H *= 2;
     d.P /= 2;
     d.hs = 1;
@@ -178,7 +183,11 @@ int plan(const ssd_desc_t* s, Plan* p, bool tight = false) {
     const int64_t st_bytes = max_chunks * d.H * d.Ppad * d.Npad * 4;
     const int64_t fb = s_bytes ? (tight ? st_bytes : std::max(st_bytes, kFwdTiles)) / (int64_t)s_bytes : units;
     const int64_t bb = kBwdTiles / (int64_t)(p->nslices * unit_bytes + s_bytes);
-    p->f32_fbatch = (int)std::max<int64_t>(1, std::min({units, fb, (int64_t)INT32_MAX}));
+    // the grids are on one axis of 2^32 threads: per unit the scan's heads of a group and 64-column parts of a head,
+    // and the S tiles' waves
+    const int64_t unit_threads = std::max<int64_t>((int64_t)d.hpg * ((d.P + 63) / 64) * 64 * ((d.Qpad / 32 + 1) / 2),
+                                                   (int64_t)(unit_bytes / 4096 + 3) / 4 * 256);
+    p->f32_fbatch = (int)std::max<int64_t>(1, std::min({units, fb, (int64_t)UINT32_MAX / unit_threads}));
     p->f32_bbatch = (int)std::max<int64_t>(1, std::min(units, bb));
     int64_t nhs = 2048 / (units * 2 * (d.Qpad / 32)) - 1;
     nhs = std::min<int64_t>(std::max<int64_t>(nhs, 1), d.hpg);

@@ -17,6 +17,8 @@
 //   F: lane = output token l, registers over source tokens s   (S of the scan: M x)
 //   R: lane = s, registers over l                              (S of the backward, dS: M^T dy, dS^T C)
 // Tile (lt, st), st <= lt, of a unit (chunk, group) is number lt (lt + 1) / 2 + st.
+#include <algorithm>
+
 #include "ssd_launch.h"
 #include "ssd_stage.h"
 #include "ssd_tile.h"
@@ -898,20 +900,18 @@ bool f32_self(const SsdDims& d) { return d.hpg == 1 && d.Npad == 32; }
 // `few`: a wave per tile.
 template <int PT, int NT>
 static hipError_t f32_scan_t(const SsdDims& d, const SsdBufs& b, F32Args a, float* y, bool few, hipStream_t s) {
-  const int units = d.max_chunks * d.G, nph = (d.P + 32 * PT - 1) / (32 * PT), nl = d.Qpad / 32;
+  const int64_t units = (int64_t)d.max_chunks * d.G;
+  const int nph = (d.P + 32 * PT - 1) / (32 * PT), nl = d.Qpad / 32;
   const size_t lds = lds_f32_scan(d, PT);
   const dim3 thr(64 * (few ? nl : (nl + 1) / 2));
-  if (f32_self(d)) {
-    ensure_lds(k_f32_scan<PT, NT, NT == 1>, lds);
-    hipLaunchKernelGGL((k_f32_scan<PT, NT, NT == 1>), dim3((unsigned)units * nph), thr, lds, s, d, a, y, nph);
-    return hipGetLastError();
-  }
-  ensure_lds(k_f32_scan<PT, NT, false>, lds);
-  for (int u0 = 0; u0 < units; u0 += b.f32_batch) {
-    const int n = min(b.f32_batch, units - u0);
-    a.unit0 = u0;
-    cb_launch<NT, true>(d, a, n, s);
-    hipLaunchKernelGGL((k_f32_scan<PT, NT, false>), dim3((unsigned)n * d.hpg * nph), thr, lds, s, d, a, y, nph);
+  const bool self = f32_self(d);
+  auto k = self ? k_f32_scan<PT, NT, NT == 1> : k_f32_scan<PT, NT, false>;
+  ensure_lds(k, lds);
+  for (int64_t u0 = 0; u0 < units; u0 += b.f32_batch) {
+    const int n = (int)std::min<int64_t>(b.f32_batch, units - u0);
+    a.unit0 = (int)u0;
+    if (!self) cb_launch<NT, true>(d, a, n, s);
+    hipLaunchKernelGGL(k, dim3((unsigned)n * d.hpg * nph), thr, lds, s, d, a, y, nph);
   }
   return hipGetLastError();
 }

@@ -152,6 +152,20 @@ def test_fp32_workspaces_hold_no_tiles_that_nothing_reads(capi):
     assert grown < chunks * unit + (64 << 20)
 
 
+@pytest.mark.parametrize("kw,whole", [
+    (dict(batch=32000, seqlen=64, nheads=65, ngroups=1, chunk=64), False),    # 2.08 M chunk-heads
+    (dict(batch=32300, seqlen=64, nheads=65, ngroups=1, chunk=64), True),     # 2^32 threads of 1024 a kernel head
+    (dict(batch=160, seqlen=8192, nheads=8, ngroups=8, chunk=256), False),    # 15.0 GiB of dS tiles
+    (dict(batch=176, seqlen=8192, nheads=8, ngroups=8, chunk=256), True),     # 16.5 GiB
+])
+def test_wide_heads_run_whole_past_the_limits_of_pairs(capi, kw, whole):
+    """Told apart by the decays' factors, one row per chunk and kernel head in the forward scratch."""
+    d = _desc(capi, headdim=128, dstate=8, has_z=0, **kw)
+    states = kw["batch"] * (kw["seqlen"] // kw["chunk"]) * kw["nheads"]
+    fwd = capi.load().ssd_workspace_bytes(ctypes.byref(d), capi.SSD_WS_FWD_SCRATCH)
+    assert fwd == states * (128 * 32 * 4 + (1 if whole else 2) * kw["chunk"] * 4)
+
+
 def test_workspace_sizes(capi):
     lib = capi.load()
     d = _desc(capi)
