@@ -14,7 +14,7 @@ import test_gpu_parity as tp
 from conftest import gpu_available
 from oracle.inputs import SsdShape, make_inputs
 from oracle.ssd_extended import ssd_combined
-from ssd_testlib import assert_close, rel_err
+from ssd_testlib import assert_close
 
 pytestmark = [pytest.mark.gpu,
               pytest.mark.skipif(not gpu_available(), reason="needs an MI355X (HIP device)")]
@@ -67,8 +67,7 @@ def test_shapes(P, H, N, Q, L, cu, monkeypatch):
 @pytest.mark.parametrize("Q", [64, 192, 256])
 def test_growing_and_steep_heads(Q, monkeypatch):
     """A head with A > 0 and one past every decay's range, whose chunks the general path leaves to its exact fixup:
-    1e-2 of the fp64 oracle, or the general path's own error where that is larger (dA of the growing head is a sum
-    that cancels; the two paths' roundings there differ by the order of sums only, hence the factor 1.25)."""
+    every gradient, of either path, within the flat 1e-2 of the fp64 oracle (they land at 3.7e-3 and below)."""
     shape = SsdShape(2, 576, 8, 64, 8, 64, Q)
 
     def grow(inp):
@@ -82,7 +81,8 @@ def test_growing_and_steep_heads(Q, monkeypatch):
     out, fin = ssd_combined(t["x"], t["dt"], t["A"], t["B"], t["C"], Q, D=t["D"], initial_states=t["init"])
     torch.autograd.backward([out, fin], [inp["dy"].to(BF).double(), inp["dfinal"].double()])
     for k, v in t.items():
-        assert_close("d" + k, head[k], v.grad, max(1e-2, 1.25 * rel_err(general[k], v.grad)))
+        assert_close("d" + k, head[k], v.grad, 1e-2)
+        assert_close("general d" + k, general[k], v.grad, 1e-2)
 
 
 @pytest.mark.parametrize("exact", [False, True], ids=["drop_beta_dA", "exact_dA"])
