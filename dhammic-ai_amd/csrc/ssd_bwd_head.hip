@@ -20,11 +20,13 @@
 // Decays are exact (exp and both clamps per element; 36 tiles x 16 exps per lane and head hide beside the MFMAs),
 // so no (chunk, head) needs the factorised kernels' fixup.
 //
-// At B=4 L=4096 H=32 P=64 N=128 chunk 256 (2048 blocks, one per CU): 352 us, against 722 us of the column and
-// row kernels (355 + 367); the whole backward of the reference scan there 317 us against 725 (chunk 64: 483 / 788,
-// chunk 256 with N = 16: 187 / 459; 64 tokens of 4 heads: 91 / 96). A block's 0.37 MB take 150 us of that at the
-// copy rate; the rest is the block's own chain load -> tiles -> dS exchange with 8 waves and no second block beside
-// it (LDS 150 KB, 256 VGPRs): waves wait 47% of their cycles, the MFMA pipes run 14%.
+// At B=4 L=4096 H=32 P=64 N=128 chunk 256 (2048 blocks, one per CU), against the column and row kernels: the reference
+// scan (MODE 0) 274 us / 342 + 323, its whole backward 317 / 725 (chunk 64: 483 / 788, chunk 256 with N = 16: 187 / 459;
+// 64 tokens of 4 heads: 91 / 96); the trapezoidal scan with the gamma path's decay gradient (MODE 3) 338 us / 357 + 372.
+// A block's 0.37 MB take 150 us of that at the copy rate; the rest is the block's own chain load -> tiles -> dS exchange
+// with 8 waves and no second block beside it (LDS 150 KB, 256 VGPRs): waves wait 47% of their cycles, the MFMA pipes run
+// 14% (MODE 3). With NT = 4 the 256 VGPRs do not quite do: 4 and 6 spill in MODE 0 and 1 (PT = 2), 12 and 21 in MODE 3
+// (PT = 1 and 2) where the B rows of phase 2 are loaded late (LATE), 84 and 122 where they are in flight through 1c.
 #include "ssd_launch.h"
 #include "ssd_tile.h"
 
@@ -139,7 +141,8 @@ __device__ __forceinline__ bf16x8 head_lo_frag(uint2 u) {
 
 // MODE: 0 plain, 1 trapezoidal (strictly causal, D per token; the diagonal of dS is gamma x.dy), 3 the same with
 // the gamma path's decay gradient (G and E weighted by gamma, the Y_off term over its states).
-template <int PT, int NT, int MODE>
+// LATE: phase 2's B rows are loaded after 1c, not in flight through it.
+template <int PT, int NT, int MODE, bool LATE>
 __global__ void __launch_bounds__(512, 2) k_bwd_head(SsdDims d, BwdHeadArgs a) {
   constexpr int PP = 32 * PT, NP = 32 * NT, PPI = tpitch<PP>(), NPI = tpitch<NP>(), TPI = tpitch<32>();
   constexpr bool TZ = MODE != 0;
@@ -418,7 +421,7 @@ __global__ void __launch_bounds__(512, 2) k_bwd_head(SsdDims d, BwdHeadArgs a) {
   }
 
   // ---- 1c ----
-  rC.load(Bg, brow, ci.len, d.N);  // phase 2's B rows
+  if (!LATE) rC.load(Bg, brow, ci.len, d.N);  // phase 2's B rows
   if (live) {
     relane();
     const int l = 32 * st + l32;
@@ -455,6 +458,7 @@ __global__ void __launch_bounds__(512, 2) k_bwd_head(SsdDims d, BwdHeadArgs a) {
     osum = add_xor32(osum);
     if (hh == 0 && l < ci.len) a.dcs_off[hq + l] = osum * et * (fabsf(csl2) < SSD_T2 ? 1.0f : 0.0f);
   }
+  if (LATE) rC.load(Bg, brow, ci.len, d.N);
   __syncthreads();  // C, dy, the states and the scalars are done with; s_dD written
   float dD0 = 0.0f;
   if (threadIdx.x < nl / 2) dD0 = s_dD[2 * threadIdx.x] + s_dD[2 * threadIdx.x + 1];
@@ -537,18 +541,22 @@ size_t lds_bwd_head(const SsdDims& d) {
   }
 }
 
-template <int PT, int NT, int MODE>
+template <int PT, int NT, int MODE, bool LATE = false>
 static hipError_t bwd_head_launch(const SsdDims& d, const BwdHeadArgs& a, hipStream_t s) {
   const size_t lds = lds_bwd_head(d);
-  ensure_lds(k_bwd_head<PT, NT, MODE>, lds);
-  hipLaunchKernelGGL((k_bwd_head<PT, NT, MODE>), dim3((unsigned)d.max_chunks * d.H), dim3(2 * d.Qpad), lds, s, d, a);
+  ensure_lds(k_bwd_head<PT, NT, MODE, LATE>, lds);
+  hipLaunchKernelGGL((k_bwd_head<PT, NT, MODE, LATE>), dim3((unsigned)d.max_chunks * d.H), dim3(2 * d.Qpad), lds, s, d, a);
   return hipGetLastError();
 }
 
 template <int PT, int NT>
 static hipError_t bwd_head_t(const SsdDims& d, const BwdHeadArgs& a, hipStream_t s) {
   if (!d.trapz) return bwd_head_launch<PT, NT, 0>(d, a, s);
-  return d.gdec ? bwd_head_launch<PT, NT, 3>(d, a, s) : bwd_head_launch<PT, NT, 1>(d, a, s);
+  if (!d.gdec) return bwd_head_launch<PT, NT, 1>(d, a, s);
+  // Six or eight tiles a block: the spills of MODE 3 cost more than a late load (782 -> 768 us, the whole call at chunk
+  // 256); two or four: the late load does (chunk 64 1095 / 1108, chunk 128 896 / 900).
+  if (NT == 4 && d.Qpad > 128) return bwd_head_launch<PT, NT, 3, NT == 4>(d, a, s);
+  return bwd_head_launch<PT, NT, 3>(d, a, s);
 }
 
 hipError_t launch_bwd_head(const SsdDims& d, const SsdBufs& b, const SsdIn& in, const void* dy, void* dx, void* dB,

@@ -100,3 +100,11 @@ def test_walks_and_pair_scan_leave_room_for_two_blocks(kernels_meta):
     for (pt, nt, nb, s32), k in _variants(kernels_meta, "k_scan_fwd_chunk").items():
         if s32 and (nb == 1 or nb == 2 and nt < 4):
             assert k["allocated"] <= 256, (pt, nt, nb, k["allocated"])
+
+
+def test_head_kernel_spills_little(kernels_meta):
+    """k_bwd_head<PT, NT, MODE, LATE>: no spills but a few registers with NT = 4, whose dC / dB accumulators and dS
+    tiles alone take 128 of the 256 (more only in the variant of the shortest chunks' MODE 3)."""
+    for (pt, nt, mode, late), k in _variants(kernels_meta, "k_bwd_head").items():
+        if mode != 3 or late or nt < 4:
+            assert k[".vgpr_spill_count"] <= (24 if nt == 4 else 0), (pt, nt, mode, k[".vgpr_spill_count"])
