@@ -25,7 +25,7 @@ ARCH = "gfx950"
 CFLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-mcode-object-version=5",
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable", "-Wno-unused-parameter",
-    # packed fp32 VALU ops are kept out of every kernel on this pool
+    # packed fp32 VALU ops are kept out of every kernel (some of their forms have given wrong results)
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     f"-I{PKG.parent / 'include'}",
 ]
@@ -33,7 +33,7 @@ CFLAGS = [
 # Files whose loops carry an MFMA accumulator through VALU code (the state walks' chunk-end update, the
 # forward scan's per-head epilogue): with the default AGPR form the compiler copies the accumulator
 # between AGPRs and VGPRs on every iteration (16 + 16 moves per 32 x 32 tile); the VGPR form keeps it in
-# place. Not global: the fp32 forward kernel spills with it.
+# place. Not global: the other files are not measured with it.
 MFMA_VGPR_FORM = {"ssd_state_fused.hip", "ssd_scan_fwd_fact.hip"}
 
 

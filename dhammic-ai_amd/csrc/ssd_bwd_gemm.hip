@@ -222,18 +222,6 @@ __global__ void __launch_bounds__(512, (GemmCfg<PT, NT>::kWaves)) k_bwd_gemm(Ssd
             rl, ok ? (int)hin_lo_off(PP, 32 * (nh * NTW + q), 16 * kk) + ln * 8 : SSD_BUF_SIZE, 0, 0));
       }
   };
-  // e4m3 bytes -> the bf16 MFMA operand: the residual (the conversion multiplies by its scale)
-  auto lo_frag = [](uint2 u) {
-    bf16x8 f;
-    constexpr float sc = 1.0f / SSD_LO_SCALE;
-    const ssd_bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, sc, false);
-    const ssd_bf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, sc, true);
-    const ssd_bf16x2 e = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, sc, false);
-    const ssd_bf16x2 g = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, sc, true);
-    f[0] = a[0]; f[1] = a[1]; f[2] = b[0]; f[3] = b[1]; f[4] = e[0]; f[5] = e[1]; f[6] = g[0]; f[7] = g[1];
-    return f;
-  };
-
   // head order rotated per chunk (the blocks of one chunk keep the same order, so they still share each
   // head's tiles through L2): the resident blocks then read different 128-byte columns of the 8 KB token
   // rows at any moment instead of all the same one (HBM channel spread)

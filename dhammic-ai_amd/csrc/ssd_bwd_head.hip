@@ -125,18 +125,6 @@ struct HeadState {
   }
 };
 
-// e4m3 bytes -> the bf16 MFMA operand (the states' rounding residual; the conversion multiplies by its scale)
-__device__ __forceinline__ bf16x8 head_lo_frag(uint2 u) {
-  bf16x8 f;
-  constexpr float sc = 1.0f / SSD_LO_SCALE;
-  const ssd_bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, sc, false);
-  const ssd_bf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, sc, true);
-  const ssd_bf16x2 e = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, sc, false);
-  const ssd_bf16x2 g = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, sc, true);
-  f[0] = a[0]; f[1] = a[1]; f[2] = b[0]; f[3] = b[1]; f[4] = e[0]; f[5] = e[1]; f[6] = g[0]; f[7] = g[1];
-  return f;
-}
-
 }  // namespace
 
 // MODE: 0 plain, 1 trapezoidal (strictly causal, D per token; the diagonal of dS is gamma x.dy), 3 the same with
@@ -435,7 +423,7 @@ __global__ void __launch_bounds__(512, 2) k_bwd_head(SsdDims d, BwdHeadArgs a) {
       for (int k = 0; k < 2 * PT; ++k) mfma(T, ttr_std<NP>(hinT, 16 * k, 32 * n, lane), yfr[k]);
       if (MODE != 3 && lo) {
 #pragma unroll
-        for (int k = 0; k < 2 * PT; ++k) mfma(T, head_lo_frag(lf[n][k]), yfr[k]);
+        for (int k = 0; k < 2 * PT; ++k) mfma(T, lo_frag(lf[n][k]), yfr[k]);
       }
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[n][v] = et * T[v];
@@ -445,7 +433,7 @@ __global__ void __launch_bounds__(512, 2) k_bwd_head(SsdDims d, BwdHeadArgs a) {
         for (int k = 0; k < 2 * PT; ++k) mfma(T, ttr_std<NP>(dstT, 16 * k, 32 * n, lane), yfr[k]);
         if (lo) {
 #pragma unroll
-          for (int k = 0; k < 2 * PT; ++k) mfma(T, head_lo_frag(lf[n][k]), yfr[k]);
+          for (int k = 0; k < 2 * PT; ++k) mfma(T, lo_frag(lf[n][k]), yfr[k]);
         }
       }
 #pragma unroll

@@ -169,17 +169,6 @@ __device__ __forceinline__ void bwd_rows_role(int c, int g, SSD_ROWS_PARAMS) {
     }
     if (d.trapz) s_gm = buf_ldf(rgm, (int)((lt * (int64_t)d.H + h) * 4), ok);
   };
-  // e4m3 bytes -> the bf16 MFMA operand: the residual (the conversion multiplies by its scale)
-  auto lo_frag = [](uint2 u) {
-    bf16x8 f;
-    constexpr float sc = 1.0f / SSD_LO_SCALE;
-    const ssd_bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, sc, false);
-    const ssd_bf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, sc, true);
-    const ssd_bf16x2 e = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, sc, false);
-    const ssd_bf16x2 f2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, sc, true);
-    f[0] = a[0]; f[1] = a[1]; f[2] = b[0]; f[3] = b[1]; f[4] = e[0]; f[5] = e[1]; f[6] = f2[0]; f[7] = f2[1];
-    return f;
-  };
 
   // C[t][n] at this lane's accumulator rows n (the Y_off part of the decay gradient), dC role
   const __amdgpu_buffer_rsrc_t rC = buf_rsrc(Cm + (int64_t)ci.row0 * brow + (int64_t)g * d.N);

@@ -440,6 +440,17 @@ __device__ __forceinline__ unsigned lo_pack4(float v0, float v1, float v2, float
   w = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(w, r(v2), r(v3), sc, true);
   return __builtin_bit_cast(unsigned, w);
 }
+// Eight such bytes as a bf16 MFMA operand.
+__device__ __forceinline__ bf16x8 lo_frag(uint2 u) {
+  bf16x8 f;
+  constexpr float sc = 1.0f / SSD_LO_SCALE;
+  const ssd_bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, sc, false);
+  const ssd_bf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.x, sc, true);
+  const ssd_bf16x2 c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, sc, false);
+  const ssd_bf16x2 d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u.y, sc, true);
+  f[0] = a[0]; f[1] = a[1]; f[2] = b[0]; f[3] = b[1]; f[4] = c[0]; f[5] = c[1]; f[6] = d[0]; f[7] = d[1];
+  return f;
+}
 
 struct ChunkInfo {
   int32_t row0;
