@@ -50,6 +50,18 @@ __device__ __forceinline__ void st_tile(float* __restrict__ t, int lane, const f
     *reinterpret_cast<floatx4*>(p + 256 * q) = floatx4{f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]};
 }
 
+// Sum in pairs: the rounding of four additions, not of sixteen (the decay gradient is a difference of such sums).
+__device__ __forceinline__ float sum16(const float (&a)[16]) {
+  float s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) s[i] = a[2 * i] + a[2 * i + 1];
+#pragma unroll
+  for (int w = 4; w > 0; w >>= 1)
+#pragma unroll
+    for (int i = 0; i < w; ++i) s[i] = s[2 * i] + s[2 * i + 1];
+  return s[0];
+}
+
 // Rows [0, nrows) (valid below len) x [0, W) columns (valid below width) of a row-major tensor into LDS
 // (pitch floats per row), zeros elsewhere. Masked buffer loads, eight pieces per thread in flight; ssd_stage.h has
 // the addresses.
@@ -543,11 +555,11 @@ __global__ void __launch_bounds__(256, 2) k_f32_col(SsdDims d, SsdBufs bf, F32Ar
           const float L = ok ? exp_clamp(dd) : 0.0f;
           const float m = S[v] * L, dm = P[v] * dt_s;
           G[v] = dm * m * clamp_pass(dd);
-          gcol += G[v];
           S[v] = m;
           P[v] = dm * L;
         }
         // (rows past the chunk's length have dy = 0; their S tile rows are zero as well)
+        gcol += sum16(G);
         const float rs = half_reduce16(G, lane);
         if (!(lane & 1)) rowp[st * Qpad + 32 * lt + acc_row((l32 >> 1) & 15, lane)] = rs;
         if (h > h_lo) {
@@ -605,7 +617,7 @@ __global__ void __launch_bounds__(256, 2) k_f32_col(SsdDims d, SsdBufs bf, F32Ar
       }
       relane();
       const float cs_last = s_cs[Qpad - 1];
-      float e[16], xs[16], dpart = 0.0f;
+      float e[16], xs[16], dpart = 0.0f, d4 = 0.0f;  // (d4: of four rows)
       const __amdgpu_buffer_rsrc_t rdx = buf_rsrc(dx + xo + (int64_t)st_row * xrow);
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -624,12 +636,16 @@ __global__ void __launch_bounds__(256, 2) k_f32_col(SsdDims d, SsdBufs bf, F32Ar
           const float tx = tmp[t][v] * ws, dXv = dX[t][v] + tx;
           ev += xx * tx;
           xv += xx * dXv;
-          dpart += xx * yy;
+          d4 += xx * yy;
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dts * dXv + Dl * yy), rdx, ok ? o : SSD_BUF_SIZE, 0, 0);
         }
         e[v] = ev * dts * clamp_pass(dl);
         xs[v] = xv;
-        if ((v & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // four rows' x loads in flight at a time
+        if ((v & 3) == 3) {
+          dpart += d4;
+          d4 = 0.0f;
+          __builtin_amdgcn_sched_barrier(0);  // four rows' x loads in flight at a time
+        }
       }
       const float er = half_reduce16(e, lane), xr = half_reduce16(xs, lane);
       const int s = 32 * st + acc_row((l32 >> 1) & 15, lane);
