@@ -457,9 +457,11 @@ k_bwd_main(SsdDims d, BwdMainArgs a, int total) {
 // Host side
 // ---------------------------------------------------------------------------
 // Shapes of the fused path; at launch it also needs 16-byte vector access
-// (d.vec_x, d.vec_bc), otherwise ssd_bwd runs the column / row kernels.
+// (d.vec_x, d.vec_bc), otherwise ssd_bwd runs the column / row kernels. The kernels address a chunk's B / C
+// rows with 32-bit byte offsets (x rows always fit: 255 rows of 65535 heads of 64 columns).
 bool bwd_main_supported(int dtype, const SsdDims& d) {
-  return dtype == 1 && d.Ppad <= 64 && d.Qpad <= 256 && d.Npad <= 128 && d.P % 8 == 0 && d.N % 8 == 0;
+  return dtype == 1 && d.Ppad <= 64 && d.Qpad <= 256 && d.Npad <= 128 && d.P % 8 == 0 && d.N % 8 == 0 &&
+         (int64_t)d.Qpad * d.G * d.N * 2 <= INT32_MAX;
 }
 
 size_t lds_bwd_main(const SsdDims& d) {

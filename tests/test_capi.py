@@ -166,6 +166,14 @@ def test_wide_heads_run_whole_past_the_limits_of_pairs(capi, kw, whole):
     assert fwd == states * (128 * 32 * 4 + (1 if whole else 2) * kw["chunk"] * 4)
 
 
+def test_fused_backward_stays_below_32_bit_row_offsets(capi):
+    """A chunk of B / C rows past 2 GiB takes the general kernels, told by the absence of dS tiles."""
+    lib = capi.load()
+    size = lambda G: lib.ssd_workspace_bytes(ctypes.byref(_desc(  # noqa: E731
+        capi, batch=1, seqlen=256, nheads=G, ngroups=G, headdim=8, dstate=128, has_z=0)), capi.SSD_WS_BWD_SCRATCH) / G
+    assert size(32767) > size(32769) + 16 * 4096 * 4
+
+
 def test_workspace_sizes(capi):
     lib = capi.load()
     d = _desc(capi)

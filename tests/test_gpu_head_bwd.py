@@ -120,3 +120,32 @@ def test_captured_backward_replays(monkeypatch):
         torch.cuda.synchronize()
         for a, b in zip(got, want):
             assert torch.equal(a, b)
+
+
+def test_more_groups_than_32_bit_offsets_reach(monkeypatch):
+    """33 000 heads with B and C of their own, 128 columns each: a chunk's rows span 2.2 GB, so the general kernels run.
+    The gradients of the first and last heads are those of the call on those heads alone, to the two paths' roundings."""
+    import kernels
+    monkeypatch.delenv("SSD_ROW_KERNEL", raising=False)
+    H, L, k = 33000, 256, 4
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    full = {"x": rnd(1, L, H, 8).to(BF), "dt": torch.rand(1, L, H, generator=g, device=DEV) * 0.1,
+            "A": -torch.rand(H, generator=g, device=DEV) * 4 - 1}
+    for n in "BC":
+        full[n] = torch.empty(1, L, H, 128, dtype=BF, device=DEV)
+        for t in range(0, L, 32):
+            full[n][:, t:t + 32] = rnd(1, 32, H, 128).div_(128 ** 0.5)
+    dy = rnd(1, L, H, 8).to(BF)
+
+    def grads(t, d):
+        t = {n: v.requires_grad_(True) for n, v in t.items()}
+        y = kernels.ssd_scan_combined(t["x"], t["dt"], t["A"], t["B"], t["C"], 256)
+        return dict(zip(t, torch.autograd.grad(y, list(t.values()), d)))
+
+    got = grads(full, dy)
+    for lo in (0, H - k):
+        cut = lambda n, v: (v[lo:lo + k] if n == "A" else v[:, :, lo:lo + k]).detach().contiguous()  # noqa: E731,B023
+        want = grads({n: cut(n, v) for n, v in full.items()}, cut("dy", dy))
+        for n in want:
+            assert_close(f"d{n} from head {lo}", cut(n, got[n]), want[n], 1e-2)
