@@ -580,12 +580,12 @@ static void state_fused_launch(const SsdDims& d, const SsdBufs& b, const bf16* u
   const int units = d.H * d.nseq;
   const int per_walk = nsplit == 1 ? units : (units + 7) / 8 * 16;
   const dim3 grid(per_walk * (w2.fac ? 2 : 1));
-  // One block per CU (by asking for more than half its LDS) where each has a CU to itself anyway, and for packed
-  // sequences up to three times that: the longest walks, which start first, are what the launch waits for, and a second
-  // block slows them (65 536 tokens of 32 heads, forward and backward, one / two: 15 sequences 1414 / 1435 us, 24
-  // 1431 / 1443; 32 768 tokens of 64 heads in 15, 960 walks: 1239 / 1224).
+  // One block per CU (by asking for more than half its LDS) for packed sequences of up to three walks a CU: the longest
+  // walks, which start first, are what the launch waits for, and a second block slows them (65 536 tokens of 32 heads,
+  // forward and backward, one / two: 15 sequences 1414 / 1435 us, 24 1431 / 1443; 32 768 tokens of 64 heads in 15, 960
+  // walks: 1239 / 1224).
   const size_t lone = 81 * 1024, need = Cfg::bytes(!FWD);
-  const size_t lds = (int)grid.x <= (d.varlen ? 768 : 256) && need < lone ? lone : need;
+  const size_t lds = d.varlen && grid.x > 256 && grid.x <= 768 && need < lone ? lone : need;
   ensure_lds(k_state_fused<PT, NT, FWD>, lds);
   hipLaunchKernelGGL((k_state_fused<PT, NT, FWD>), grid, dim3(Cfg::NTHR), lds, s, d, b.chunks, b.seq_chunk0,
                      b.seq_order, b.cs, fac, u, v, hst, hlo, hin_in, s_in, s_out, state_bf16, b.dtot_part, nsplit,
