@@ -25,7 +25,7 @@
 // 64 tokens of 4 heads: 91 / 96); the trapezoidal scan with the gamma path's decay gradient (MODE 3) 338 us / 357 + 372.
 // A block's 0.37 MB take 150 us of that at the copy rate; the rest is the block's own chain load -> tiles -> dS exchange
 // with 8 waves and no second block beside it (LDS 150 KB, 256 VGPRs): waves wait 47% of their cycles, the MFMA pipes run
-// 14% (MODE 3). With NT = 4 the 256 VGPRs do not quite do: 4 and 6 spill in MODE 0 and 1 (PT = 2), 12 and 21 in MODE 3
+// 14%. With NT = 4 the 256 VGPRs do not quite do: 4 and 6 spill in MODE 0 and 1 (PT = 2), 12 and 21 in MODE 3
 // (PT = 1 and 2) where the B rows of phase 2 are loaded late (LATE), 84 and 122 where they are in flight through 1c.
 #include "ssd_launch.h"
 #include "ssd_tile.h"

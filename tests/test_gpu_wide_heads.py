@@ -84,6 +84,32 @@ def test_rows_off_the_16_byte_grid():
     assert all(rel_err(a, b) <= TOL[BF] for a, b in zip(*outs)), [rel_err(a, b) for a, b in zip(*outs)]
 
 
+@pytest.mark.parametrize("copies", [True, False], ids=["copied", "in place"])
+@pytest.mark.parametrize("P,G,N,z", [(128, 3, 32, True), (96, 1, 64, False)])
+def test_rows_off_the_grid_are_copied(P, G, N, z, copies, monkeypatch):
+    """x, B, C, z and dy at storage offset 1: the Python layer copies them onto the grid, with the aligned call's bits;
+    without the copies (as a caller of the C ABI has it) the general kernels run on the pairs."""
+    import kernels
+    from kernels import ssd_scan as ks
+    if not copies:
+        monkeypatch.setattr(ks, "_on_grid", lambda *t: t)
+    inp = make_inputs(SsdShape(2, 200, 3, P, G, N, 64), seed=9, with_z=z)
+    off = lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)  # noqa: E731
+    outs = []
+    for place in (lambda t: t, off):
+        t = {k: place(inp[k].to(DEV, BF)) if k in ("x", "B", "C", "z") else inp[k].to(DEV)
+             for k in ("x", "dt", "A", "B", "C", "D") + (("z",) if z else ())}
+        t = {k: v.requires_grad_(True) for k, v in t.items()}
+        w = torch.ones(3 * P, device=DEV) if z else None
+        y = kernels.ssd_scan_combined(*[t[k] for k in ("x", "dt", "A", "B", "C")], 64, D=t["D"], z=t.get("z"),
+                                      norm_weight=w)
+        outs.append([y] + list(torch.autograd.grad(y, list(t.values()), place(inp["dy"].to(DEV, BF)))))
+    if copies:
+        assert all(torch.equal(u, v) for u, v in zip(*outs))
+    else:
+        assert all(rel_err(u, v) <= TOL[BF] for u, v in zip(*outs)), [rel_err(u, v) for u, v in zip(*outs)]
+
+
 def test_noalloc_forward_on_both_sides_of_the_pairs_limit():
     """A forward whose pairs fit the 64 MiB scratch, and one that fits only with whole heads, which
     ssd_fwd_noalloc then runs: the second agrees with ssd_fwd's pairs to bf16 rounding."""
